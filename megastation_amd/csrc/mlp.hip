@@ -7,11 +7,14 @@
 // GEMM: C[M][N] = sum_k A(i,k) B(k,j), A(i,k) = A[i*sai + k*sak],
 // B(k,j) = B[k*sbk + j*sbj] (any transpose through the strides), C row-major
 // FP32 (ldc) and/or BF16 with an epilogue: + bias[j], then GELU (tanh form)
-// or identity. 64 x 64 tiles per 256-thread workgroup, K in steps of 32
-// staged through LDS as BF16 (the next step's vectors loaded during this
-// step's products); each wave owns a 32 x 32 quarter (2 x 2
-// v_mfma_f32_16x16x32_bf16 tiles). Small M x N grids split K over more
-// workgroups and add the partial sums in a second kernel.
+// or identity. Operands whose rows load in whole vectors go to gemm_direct
+// (registers, K split over the waves of a workgroup). The others (rows off
+// the 16-byte grid, both strides other than 1, more than 8 splits) take
+// gemm_bf16: 64 x 64 tiles per 256-thread workgroup, K in steps of 32 staged
+// through LDS as BF16 (the next step's vectors loaded during this step's
+// products), each wave a 32 x 32 quarter (2 x 2 v_mfma_f32_16x16x32_bf16
+// tiles), small grids splitting K over more workgroups and adding the partial
+// sums in a second kernel.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -147,6 +150,162 @@ __global__ __launch_bounds__(256) void gemm_bf16(const __bf16* __restrict__ A, i
       }
 }
 
+// ---- Direct GEMM: operands straight from global memory into registers -------
+//
+// One workgroup owns one (16 FM) x (16 FN) tile of C. Where the staged kernel
+// splits K, a workgroup's waves take the splits' ranges and the partial tiles
+// are added in split order through LDS (no second kernel, no workspace): every
+// output is the same chain of MFMAs and sums, bit for bit. The shapes of the network (M 60-2112, N 512-2112, K 512-2112) are
+// bound by latency, not by the matrix cores or L2: a staged tile paid two
+// barriers and a transposing 2-byte LDS scatter per 32-wide step on one wave a
+// SIMD, here a wave keeps PD steps of both operands in flight and no wave waits
+// for another before the end.
+//
+// An operand whose K index is the unit-stride one (KF) gives a lane its 8
+// consecutive K values as one 16-byte load per 16 rows. One whose row index is
+// (the weights' W[k][j], the transposed activations of dW) is loaded as F
+// consecutive rows of 8 K lines and the F fragments are put together with byte
+// permutes: fragment f then holds rows F*i + f instead of 16 f + i, which the
+// epilogue's row map undoes. Both operands use K = 8 (lane / 16) + v, the
+// order the MFMA sums over does not matter otherwise.
+
+template <int F, bool KF>
+struct GemmRaw {
+  static constexpr int W = KF ? 4 * F : 8 * (F / 2);  // words a lane holds
+  uint32_t w[W];
+};
+
+// Rows clamped to the last ones (their products are not stored); K lines past
+// K read as zero in the tail step.
+template <int F, bool KF, bool TAIL>
+__device__ __forceinline__ void gemm_load(GemmRaw<F, KF>& o, const __bf16* __restrict__ P,
+                                          int64_t stride, uint32_t r0, uint32_t R, uint32_t k0,
+                                          uint32_t K, int i16, int q4) {
+  if constexpr (KF) {
+    const uint32_t k = k0 + 8 * q4;
+    const bool in = !TAIL || k < K;  // K % 8 == 0
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const uint32_t r = min(r0 + 16u * f + i16, R - 1);
+      uint4 v = *reinterpret_cast<const uint4*>(P + (int64_t)r * stride + (in ? k : 0u));
+      if (TAIL && !in) v = uint4{0, 0, 0, 0};
+      o.w[4 * f] = v.x, o.w[4 * f + 1] = v.y, o.w[4 * f + 2] = v.z, o.w[4 * f + 3] = v.w;
+    }
+  } else {
+    const uint32_t r = min(r0 + (uint32_t)F * i16, R - F);  // R % F == 0
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const uint32_t k = k0 + 8 * q4 + v;
+      const bool in = !TAIL || k < K;
+      const __bf16* p = P + (int64_t)(in ? k : 0u) * stride + r;
+      if constexpr (F == 4) {
+        uint2 x = *reinterpret_cast<const uint2*>(p);
+        if (TAIL && !in) x = uint2{0, 0};
+        o.w[2 * v] = x.x, o.w[2 * v + 1] = x.y;
+      } else {
+        uint32_t x = *reinterpret_cast<const uint32_t*>(p);
+        if (TAIL && !in) x = 0;
+        o.w[v] = x;
+      }
+    }
+  }
+}
+
+template <int F, bool KF>
+__device__ __forceinline__ v8bf gemm_frag(const GemmRaw<F, KF>& o, int f) {
+  uint4 r;
+  if constexpr (KF) {
+    r = uint4{o.w[4 * f], o.w[4 * f + 1], o.w[4 * f + 2], o.w[4 * f + 3]};
+  } else {
+    // rows F i + f: half f % 2 of word f / 2 of each K line, two lines a word
+    const uint32_t sel = f % 2 ? 0x07060302u : 0x05040100u;
+    constexpr int H = F / 2;
+    const int h = f / 2;
+    r = uint4{__builtin_amdgcn_perm(o.w[H * 1 + h], o.w[H * 0 + h], sel),
+              __builtin_amdgcn_perm(o.w[H * 3 + h], o.w[H * 2 + h], sel),
+              __builtin_amdgcn_perm(o.w[H * 5 + h], o.w[H * 4 + h], sel),
+              __builtin_amdgcn_perm(o.w[H * 7 + h], o.w[H * 6 + h], sel)};
+  }
+  return __builtin_bit_cast(v8bf, r);
+}
+
+template <int FM, int FN, bool AKF, bool BKF>
+__global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A, int64_t sa,
+                                                   const __bf16* __restrict__ B, int64_t sb,
+                                                   uint32_t M, uint32_t N, uint32_t K,
+                                                   const float* __restrict__ bias, int act,
+                                                   float* __restrict__ Cf,
+                                                   __bf16* __restrict__ Cb, uint32_t ldc,
+                                                   float beta, int steps) {
+  constexpr int GM = 16 * FM, GN = 16 * FN, LD = GN + 4, PD = 3;  // 6: no faster
+  extern __shared__ float red[];  // [SK][GM][LD]
+  const int lane = threadIdx.x & 63, i16 = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int SK = blockDim.x >> 6;
+  const uint32_t m0 = blockIdx.y * GM, n0 = blockIdx.x * GN;
+  const int full = K / 32, first = wave * steps;
+  const int n = min(full - first, steps);  // this wave's whole steps
+  v4f acc[FM][FN] = {};
+  GemmRaw<FM, AKF> ra[PD];
+  GemmRaw<FN, BKF> rb[PD];
+  auto load = [&](int d, int s) {
+    const uint32_t k0 = 32u * (first + s);
+    gemm_load<FM, AKF, false>(ra[d], A, sa, m0, M, k0, K, i16, q4);
+    gemm_load<FN, BKF, false>(rb[d], B, sb, n0, N, k0, K, i16, q4);
+  };
+  auto mul = [&](int d) {
+    v8bf a[FM], b[FN];
+#pragma unroll
+    for (int f = 0; f < FM; ++f) a[f] = gemm_frag<FM, AKF>(ra[d], f);
+#pragma unroll
+    for (int f = 0; f < FN; ++f) b[f] = gemm_frag<FN, BKF>(rb[d], f);
+#pragma unroll
+    for (int x = 0; x < FM; ++x)
+#pragma unroll
+      for (int y = 0; y < FN; ++y)
+        acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[x], b[y], acc[x][y], 0, 0, 0);
+  };
+  if (n > 0) {
+    // the ring's loads always run (clamped to the last step): no branch
+    // between them, so every wait is exact
+#pragma unroll
+    for (int d = 0; d < PD; ++d) load(d, min(d, n - 1));
+    int s = 0;
+    for (; s + PD <= n; s += PD) {
+#pragma unroll
+      for (int d = 0; d < PD; ++d) {
+        mul(d);
+        load(d, min(s + d + PD, n - 1));
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < PD - 1; ++d)
+      if (s + d < n) mul(d);
+  }
+  if (K % 32 && wave == SK - 1) {  // the tail step ends the last range
+    gemm_load<FM, AKF, true>(ra[0], A, sa, m0, M, 32u * full, K, i16, q4);
+    gemm_load<FN, BKF, true>(rb[0], B, sb, n0, N, 32u * full, K, i16, q4);
+    mul(0);
+  }
+  // D lane l, reg r = fragment row 4 (l / 16) + r, column l % 16
+#pragma unroll
+  for (int x = 0; x < FM; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = AKF ? 16 * x + 4 * q4 + r : FM * (4 * q4 + r) + x;
+      float* o = red + ((size_t)wave * GM + i) * LD;
+#pragma unroll
+      for (int y = 0; y < FN; ++y) o[BKF ? 16 * y + i16 : FN * i16 + y] = acc[x][y][r];
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < GM * GN; e += blockDim.x) {
+    const uint32_t i = e / GN, j = e % GN;
+    float s = red[(size_t)i * LD + j];
+    for (int w = 1; w < SK; ++w) s += red[((size_t)w * GM + i) * LD + j];
+    if (m0 + i < M && n0 + j < N) gemm_out(s, m0 + i, n0 + j, bias, act, Cf, Cb, ldc, beta);
+  }
+}
+
 // Sum of the K splits (in split order) and the epilogue.
 __global__ void gemm_reduce(const float* __restrict__ part, uint32_t splits, uint32_t M,
                             uint32_t N, const float* __restrict__ bias, int act,
@@ -170,20 +329,49 @@ __global__ void act_backward(const float* __restrict__ dY, const float* __restri
   if (dZf) dZf[i] = g;
 }
 
-// db[j] = sum_i dZ[i][j] (FP32): 64 columns per workgroup, the rows split
-// over 4 waves (coalesced row segments), partial sums added through LDS.
-__global__ __launch_bounds__(256) void col_sum(const float* __restrict__ dZ,
-                                               float* __restrict__ db, uint32_t M, uint32_t N) {
-  __shared__ float part[4][64];
-  const uint32_t j = blockIdx.x * 64 + (threadIdx.x & 63);
-  const uint32_t w = threadIdx.x >> 6;
-  float s = 0.f;
-  if (j < N)
-    for (uint32_t i = w; i < M; i += 4) s += dZ[(uint64_t)i * N + j];
-  part[w][threadIdx.x & 63] = s;
+// db[j] = sum_i dZ[i][j] (FP32) as four running sums over the rows i % 4,
+// added pairwise. 16 columns per workgroup (64-byte row segments): all 1024
+// threads bring 1024 rows into LDS at once, so the rows' HBM latency is paid
+// once per 1024, and one wave then runs the 64 chains from LDS. Walking the
+// rows in global memory, one chain of M / 4 loads a thread on N / 64
+// workgroups, took 79 us at 1092 x 1056 (4.6 MB).
+constexpr int CS_COLS = 16, CS_ROWS = 1024, CS_THREADS = 1024;
+__global__ __launch_bounds__(CS_THREADS) void col_sum(const float* __restrict__ dZ,
+                                                      float* __restrict__ db, uint32_t M,
+                                                      uint32_t N) {
+  __shared__ float rows[CS_ROWS][CS_COLS + 1];
+  __shared__ float part[4][CS_COLS];
+  constexpr int LANES = CS_THREADS / CS_COLS, PER = CS_ROWS / LANES;
+  const uint32_t c = threadIdx.x % CS_COLS, w = threadIdx.x / CS_COLS;
+  const uint32_t j = blockIdx.x * CS_COLS + c;
+  float s = 0.f;  // threads of wave 0: rows i % 4 == w of column c
+  for (uint32_t i0 = 0; i0 < M; i0 += CS_ROWS) {
+    const uint32_t n = min((uint32_t)CS_ROWS, M - i0);
+    float v[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const uint32_t r = min(w + q * LANES, n - 1);
+      v[q] = dZ[(uint64_t)(i0 + r) * N + min(j, N - 1)];
+    }
+    __syncthreads();  // the chains are done with the previous rows
+#pragma unroll
+    for (int q = 0; q < PER; ++q) rows[w + q * LANES][c] = v[q];
+    __syncthreads();
+    if (w < 4) {
+      uint32_t r = w;
+      for (; r + 60 < n; r += 64) {
+        float x[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) x[q] = rows[r + 4 * q][c];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s += x[q];
+      }
+      for (; r < n; r += 4) s += rows[r][c];
+    }
+  }
+  if (w < 4) part[w][c] = s;
   __syncthreads();
-  if (w == 0 && j < N) db[j] = (part[0][threadIdx.x] + part[1][threadIdx.x]) +
-                                (part[2][threadIdx.x] + part[3][threadIdx.x]);
+  if (w == 0 && j < N) db[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
 }
 
 // Gradient (y - t)/M of the MSE loss 0.5/M * sum (y - t)^2.
@@ -219,6 +407,41 @@ uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t)
 
 }  // namespace
 
+// An operand the direct kernel can load in whole vectors: K unit-stride with
+// 16-byte rows, or rows unit-stride in pieces of f.
+bool direct_kf(const __bf16* p, int64_t sr, int64_t sk, uint32_t K) {
+  return sk == 1 && sr % 8 == 0 && K % 8 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+}
+bool direct_rf(const __bf16* p, int64_t sr, int64_t sk, uint32_t R, uint32_t f) {
+  return sr == 1 && sk % f == 0 && R % f == 0 && reinterpret_cast<uintptr_t>(p) % (2 * f) == 0;
+}
+
+template <int FM, int FN, bool AKF, bool BKF>
+hipError_t direct_run(const MlpGemm& g, uint32_t sk, uint32_t kchunk, hipStream_t st) {
+  constexpr uint32_t GM = 16 * FM, GN = 16 * FN;
+  const uint32_t lds = sk * GM * (GN + 4) * sizeof(float);
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&gemm_direct<FM, FN, AKF, BKF>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  const dim3 grid((g.N + GN - 1) / GN, (g.M + GM - 1) / GM);
+  hipLaunchKernelGGL((gemm_direct<FM, FN, AKF, BKF>), grid, dim3(64 * sk), lds, st, g.A,
+                     AKF ? g.sai : g.sak, g.B, BKF ? g.sbj : g.sbk, g.M, g.N, g.K, g.bias, g.act,
+                     g.Cf, g.Cb, g.ldc, g.beta, (int)(kchunk / TK));
+  return hipGetLastError();
+}
+
+template <int FM, int FN>
+hipError_t direct_pick(const MlpGemm& g, bool akf, bool bkf, uint32_t sk, uint32_t kc,
+                       hipStream_t st) {
+  return akf ? (bkf ? direct_run<FM, FN, true, true>(g, sk, kc, st)
+                    : direct_run<FM, FN, true, false>(g, sk, kc, st))
+             : (bkf ? direct_run<FM, FN, false, true>(g, sk, kc, st)
+                    : direct_run<FM, FN, false, false>(g, sk, kc, st));
+}
+
 // K splits: enough workgroups to cover the CUs (>= 256) while every split
 // keeps at least 8 K steps. The partial sums live in the library's workspace
 // of the (device, stream) (stream_workspace): work queued on one stream runs
@@ -227,12 +450,37 @@ uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t)
 // being captured into a graph.
 hipError_t mlp_gemm(const MlpGemm& g, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
+  const bool akf = direct_kf(g.A, g.sai, g.sak, g.K), bkf = direct_kf(g.B, g.sbj, g.sbk, g.K);
+  auto fits = [&](uint32_t fm, uint32_t fn) {
+    return (akf || direct_rf(g.A, g.sai, g.sak, g.M, fm)) &&
+           (bkf || direct_rf(g.B, g.sbj, g.sbk, g.N, fn));
+  };
   const uint32_t tiles = ((g.N + TN - 1) / TN) * ((g.M + TM - 1) / TM);
   const uint32_t ksteps = (g.K + TK - 1) / TK;
   uint32_t splits = 1;
   while (tiles * splits < 256 && ksteps / (splits + 1) >= 8) ++splits;
   const uint32_t kchunk = ((ksteps + splits - 1) / splits) * TK;
   splits = (g.K + kchunk - 1) / kchunk;
+  // Direct kernel wherever both operands load in whole vectors and the splits
+  // fit a workgroup. 32 x 32 tiles spread the network's own shapes over the
+  // CUs; they read each operand once per 32 rows, so grids of 64 x 64 tiles
+  // that fill the chip several times over take those instead (L2-bound).
+  // Measured, us a call, staged kernel (+ reduce) / 32 x 32 / 64 x 64 (M x N x K,
+  // T: both operands' rows unit-stride; a call costs 8 us to issue):
+  //   273 x 512 x 2112      18.2 /  9.0 / 20.1
+  //   1092 x 512 x 2112     40.8 / 22.8 / 34.0
+  //   2112 x 512 x 1092 T    107 / 24.9 / 43.7
+  //   4368 x 512 x 512      40.0 / 26.8 / 36.2   (552 tiles of 64 x 64)
+  //   16384 x 512 x 512     81.6 / 73.4 / 59.0   (2048)
+  //   16384 x 512 x 2112     200 /  226 /  121   (2048)
+  //   2112 x 512 x 16384 T  1486 /  238 /  320   (264)
+  if (splits <= 8) {
+    const uint64_t tiles64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
+    if (tiles64 >= 1024 && fits(4, 4))
+      return direct_pick<4, 4>(g, akf, bkf, splits, kchunk, st);
+    if ((g.M + 31) / 32 <= 65535 && fits(2, 2))
+      return direct_pick<2, 2>(g, akf, bkf, splits, kchunk, st);
+  }
   float* part = nullptr;
   if (splits > 1) {
     void* w = nullptr;
@@ -263,7 +511,7 @@ hipError_t mlp_act_backward(const float* dY, const float* Z, __bf16* dZ, float* 
 
 hipError_t mlp_col_sum(const float* dZ, float* db, uint32_t M, uint32_t N, hipStream_t st) {
   if (N == 0) return hipSuccess;
-  hipLaunchKernelGGL(col_sum, dim3(blocks_for(N, 64)), dim3(256), 0, st, dZ, db, M, N);
+  hipLaunchKernelGGL(col_sum, dim3(blocks_for(N, CS_COLS)), dim3(CS_THREADS), 0, st, dZ, db, M, N);
   return hipGetLastError();
 }
 

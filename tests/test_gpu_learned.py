@@ -50,6 +50,51 @@ def test_gemm_strided_transposes(M, N, K):
             assert _rel(Cb.float().cpu().numpy(), mlp.gelu(ref)) < 1e-2
 
 
+@pytest.mark.parametrize("M,N,K", [(273, 512, 2112), (60, 512, 76), (36, 68, 24), (34, 62, 1092),
+                                   (2084, 2048, 72)])
+def test_gemm_direct_equals_staged(M, N, K):
+    """The register kernel (operands whose rows load in whole vectors) against
+    the staged one, which the same operands two bytes off the vector grid
+    take: the same chain of products per output, so equal bit for bit. Split
+    K, a K tail, tiles past the edges, a grid large enough for 64 x 64 tiles."""
+    print(f"case: gemm direct M={M} N={N} K={K}", flush=True)
+    t = torch()
+    g = t.Generator(device="cuda").manual_seed(M + K)
+    bias = t.randn(N, device="cuda", generator=g)
+
+    def off(x):  # the same values one element into a larger buffer
+        b = t.empty(x.numel() + 1, dtype=x.dtype, device="cuda")
+        b[1:] = x.reshape(-1)
+        return b[1:]
+    for a_t in (False, True):
+        for b_t in (False, True):
+            A = t.randn(M * K, device="cuda", generator=g).to(t.bfloat16)
+            B = t.randn(K * N, device="cuda", generator=g).to(t.bfloat16)
+            sa = (1, M) if a_t else (K, 1)
+            sb = (1, K) if b_t else (N, 1)
+            got = []
+            for a, b in ((A, B), (off(A), off(B))):
+                C = t.zeros(M, N, device="cuda")
+                Cb = t.zeros(M, N, dtype=t.bfloat16, device="cuda")
+                learned.gemm(a, *sa, b, *sb, M, N, K, bias=bias, act=learned.GELU, Cf=C, Cb=Cb)
+                got.append((C.cpu(), Cb.cpu()))
+            assert t.equal(got[0][0], got[1][0]) and t.equal(got[0][1], got[1][1]), (a_t, b_t)
+
+
+@pytest.mark.parametrize("M,N", [(1, 5), (3, 16), (1024, 17), (1025, 40), (2111, 33)])
+def test_col_sum_is_four_running_sums(M, N):
+    print(f"case: col_sum M={M} N={N}", flush=True)
+    t = torch()
+    X = np.random.default_rng(M).standard_normal((M, N)).astype(np.float32)
+    p = np.zeros((4, N), np.float32)
+    for i in range(M):
+        p[i % 4] += X[i]
+    Xd = t.from_numpy(X).cuda()
+    db = t.empty(N, device="cuda")
+    m._check(learned._L().mega_mlp_col_sum(m._ptr(Xd), m._ptr(db), M, N, m._stream(None)))
+    assert np.array_equal(db.cpu().numpy(), (p[0] + p[1]) + (p[2] + p[3]))
+
+
 def test_mlp_forward_backward_adam_match_oracle():
     print("case: mlp fwd/bwd/adam", flush=True)
     t = torch()
