@@ -1,6 +1,8 @@
 // Zero-forcing weights per subcarrier group (one workgroup per group, the
 // fused Gram / Gauss-Jordan / MFMA apply of zf_core.h) and the downlink
 // precoder normalisation (src/operators/beamform/beam_utils.cuh:40-80).
+#include <algorithm>
+
 #include "zf_core.h"
 
 namespace mega {
@@ -82,30 +84,64 @@ hipError_t launch_zf_ut(uint32_t U, uint32_t B, uint32_t batch, const float2* in
 }
 
 // P_g = W_g^T * (1 / max|W_g|) (beam_utils.cuh:40-80): U x B column-major in,
-// B x U column-major out.
-__global__ __launch_bounds__(256) void scale_absmax_kernel(
+// B x U column-major out. One workgroup per group (grid-stride past 65535),
+// bound by the latency of its one pass: all loads of a thread are in flight
+// together, the values wait for the maximum in LDS (rows of an odd pitch, so
+// neither the column writes nor the row reads conflict) and leave as whole
+// antenna rows. A group beyond the LDS tile takes the maximum first and reads
+// its antennas a second time, a tile at a time (bt = 0, a user count no tile
+// holds: stored straight). Storing straight from the
+// column order scattered every 8 bytes to a line of its own: 33.8 us against
+// 14.2 at 273 groups of 256 x 32 (36 MB).
+constexpr uint32_t kScaleLds = 16384 + 128;  // float2 of the tile
+__global__ __launch_bounds__(1024) void scale_absmax_kernel(
     const float2* __restrict__ in, float2* __restrict__ out, uint32_t U,
-    uint32_t B, uint32_t batch) {
-  __shared__ float sMax[256 / 64];
-  const uint32_t n = U * B;
+    uint32_t B, uint32_t batch, uint32_t bt, uint32_t pitch) {
+  __shared__ float sMax[1024 / 64];
+  extern __shared__ float sDyn[];
+  float2* tile = reinterpret_cast<float2*>(sDyn);  // [U][pitch], bt antennas
+  const uint32_t n = U * B, nt = blockDim.x;
+  const bool whole = bt >= B;
   for (uint32_t g = blockIdx.x; g < batch; g += gridDim.x) {
     const float2* x = in + (uint64_t)g * n;
     float2* o = out + (uint64_t)g * n;
     float m = 0.f;
-    for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) {
-      const float2 v = x[e];
-      m = fmaxf(m, sqrtf(v.x * v.x + v.y * v.y));
+    for (uint32_t e0 = threadIdx.x; e0 < n; e0 += 8 * nt) {
+      float2 v[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] = x[min(e0 + r * nt, n - 1)];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const uint32_t e = e0 + r * nt;
+        m = fmaxf(m, sqrtf(v[r].x * v[r].x + v[r].y * v[r].y));
+        if (whole && e < n) tile[(e % U) * pitch + e / U] = v[r];
+      }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0) sMax[threadIdx.x >> 6] = m;
     __syncthreads();
     float mx = 0.f;
-    for (uint32_t w = 0; w < (blockDim.x + 63) / 64; ++w) mx = fmaxf(mx, sMax[w]);
+    for (uint32_t w = 0; w < (nt + 63) / 64; ++w) mx = fmaxf(mx, sMax[w]);
     const float s = 1.0f / mx;
-    for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) {
-      const float2 v = x[e];
-      o[(e % U) * B + e / U] = make_float2(v.x * s - v.y * 0.f, v.x * 0.f + v.y * s);
+    if (bt == 0)
+      for (uint32_t e = threadIdx.x; e < n; e += nt) {
+        const float2 v = x[e];
+        o[(e % U) * B + e / U] = make_float2(v.x * s - v.y * 0.f, v.x * 0.f + v.y * s);
+      }
+    for (uint32_t b0 = 0; bt > 0 && b0 < B; b0 += bt) {
+      const uint32_t nb = min(bt, B - b0);
+      if (!whole) {
+        __syncthreads();  // the previous tile is out
+        for (uint32_t e = threadIdx.x; e < U * nb; e += nt)
+          tile[(e % U) * pitch + e / U] = x[(uint64_t)b0 * U + e];
+        __syncthreads();
+      }
+      for (uint32_t e = threadIdx.x; e < U * nb; e += nt) {
+        const uint32_t u = e / nb, b = e % nb;
+        const float2 v = tile[u * pitch + b];
+        o[(uint64_t)u * B + b0 + b] = make_float2(v.x * s - v.y * 0.f, v.x * 0.f + v.y * s);
+      }
     }
     __syncthreads();
   }
@@ -145,11 +181,25 @@ hipError_t launch_scale_absmax(uint32_t U, uint32_t B, uint32_t batch,
                                const float2* in, float2* out,
                                hipStream_t st) {
   if (batch == 0) return hipSuccess;
-  const uint32_t n = U * B;
-  const uint32_t threads = n >= 256 ? 256 : (n + 63) / 64 * 64;
+  const uint64_t n = (uint64_t)U * B;
+  const uint32_t threads = n >= 1024 ? 1024 : ((uint32_t)n + 63) / 64 * 64;
   const uint32_t blocks = batch < 65536 ? batch : 65535;
-  hipLaunchKernelGGL(scale_absmax_kernel, dim3(blocks), dim3(threads), 0, st, in,
-                     out, U, B, batch);
+  // antennas per LDS tile: the whole group where it fits
+  uint32_t bt = B;
+  if ((uint64_t)U * (B | 1) > kScaleLds) {
+    bt = std::min(64u, kScaleLds / U);
+    bt -= bt > 0 && bt % 2 == 0;  // an odd pitch within the tile
+  }
+  const uint32_t pitch = bt | 1;
+  const size_t lds = bt ? (size_t)U * pitch * sizeof(float2) : 0;
+  if (lds > 65536) {
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&scale_absmax_kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(scale_absmax_kernel, dim3(blocks), dim3(threads), lds, st, in, out, U, B,
+                     batch, bt, pitch);
   return hipGetLastError();
 }
 
