@@ -146,7 +146,7 @@ hipError_t launch_scale_absmax(uint32_t U, uint32_t B, uint32_t batch,
 // (and on mega_tuning_reload), sanitized to each key's accepted range; 0 is
 // the launcher's own choice except for kDetPf (default 1).
 enum TuneKey {
-  kEqKs, kEqMode, kEqSch, kEqSmt, kEqTpw, kEqXmt, kEqXreg, kEqXt, kEqXks, kPrecAcc, kDetPf,
+  kEqKs, kEqMode, kEqSch, kEqSmt, kEqTpw, kEqXmt, kEqXreg, kEqXt, kEqXks, kDetPf,
   kEqWtc, kZfNth, kZfWide, kUplinkStreams, kEqWnw, kEqWp,
   kTuneCount
 };

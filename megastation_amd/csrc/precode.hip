@@ -11,19 +11,30 @@
 // TFLOP/s dense: at 256 x 32 a slot's precode is 2.8 GFLOP against 116 MB,
 // beyond the vector ALUs' reach in the time HBM needs). The columns of a
 // group are its (symbol, subcarrier) pairs, sg * S of them, since P_g serves
-// every symbol. One workgroup per (group, block of 64 antennas) stages that
-// block of P_g in LDS once ([U][64], at most 32 KB, coalesced loads); its four
-// waves take the group's 16-column tiles in turn, each computing 32 antennas
-// (half the block; the two halves on alternate waves) x 16 columns with A operands from LDS and B operands (user symbols) gathered
-// from HBM. A complex product
-// takes real 16x16x4 steps with rows interleaved (antenna r re, r im) and K
-// interleaved (user u re, u im):
-//   A[2r][2u] = Re P, A[2r][2u+1] = -Im P, A[2r+1][2u] = Im P,
-//   A[2r+1][2u+1] = Re P;   B[2u][n] = Re x, B[2u+1][n] = Im x,
-// so D[2r][n] = Re out and D[2r+1][n] = Im out, and each lane ends with
-// whole complex outputs (rows 4*(l/16) .. +3 = two antennas) at column l%16.
-// FP32 accumulation, users in increasing order (two per step).
-#include <cstdlib>
+// every symbol. A complex product takes two real steps over four users with
+// the D rows interleaved (antenna r re, r im):
+//   A1[2r][u] = Re P, A1[2r+1][u] = Im P,  B1[u][n] = Re x
+//   A2[2r][u] = -Im P, A2[2r+1][u] = Re P, B2[u][n] = Im x,
+// so each loaded complex value is used whole and a lane ends with whole
+// complex outputs (rows 4*(l/16) .. +3 = two antennas) at column l%16. FP32
+// accumulation, users in increasing order (four per step).
+//
+// A wave holds its antennas' P_g in registers (8 NACC antennas x 4 J users: 2
+// NACC J values a lane) for every column tile of its workgroup's range, with
+// the next tile's user symbols in flight during a tile's products: no LDS and
+// no barrier, so a SIMD's two waves interleave loads, products and stores. The
+// (group, 16-column tile) pairs of an antenna block are one sequence that the
+// grid cuts into equal ranges: a range that crosses into the next group
+// reloads P there. With P in LDS and one workgroup per group and 64 antennas,
+// the four workgroups of a group gathered the same user symbols through the
+// load latency of every tile, and 1092 of them left a tail: 62.8 us a slot at
+// 256 x 32, 51 now (2.3 TB/s). What is left there: stores alone take 20 us,
+// products alone 23 (FP32 matrix rate at the clock they run at), loads 12, and
+// two waves a SIMD overlap them only in part. A finished tile's stores go out
+// among the next tile's products (56 us with the stores in one burst); more
+// tiles of user symbols in flight, or four waves of fewer antennas a SIMD (67
+// us, twice the symbol loads), do not help.
+#include <algorithm>
 
 #include "eq_core.h"
 
@@ -31,85 +42,141 @@ namespace mega {
 namespace detail {
 namespace {
 
-// 8-antenna accumulator tiles per wave: NACC = 4 (32 antennas; the two
-// halves of a workgroup's 64 antennas on alternate waves) or 8 (64).
-
-// Workgroup = (group g, block of 64 antennas ab), ab fastest, in the logical
-// order of xcd_linear: consecutive workgroups share an XCD, so a group's user
-// symbols are fetched into one L2 for all its antenna blocks, and adjacent
-// groups' partial 128-byte output lines meet in the same L2. Wave w takes the
-// 16-column tiles w, w + 4, ... A tile's user symbols (at most UMAX users,
-// two per step) are all loaded before its products, so the HBM latency is
-// paid once per tile, not once per step.
-template <int UMAX, int NACC>
-__global__ __launch_bounds__(256) void precode_mfma(const PrecodeArgs a, uint32_t nab,
-                                                   uint32_t ntile) {
-  constexpr int NKS = UMAX / 2;
-  constexpr int WPT = 8 / NACC;  // waves sharing a tile (antenna halves)
+// The antenna range [b0, b0 + 8 NACC) of this wave: NACC 8-antenna tiles, J
+// steps of four users. Workgroup order: xcd_linear, ranges of one antenna
+// block consecutive, so adjacent groups, whose output segments share 128-byte
+// lines, meet in one XCD's L2 at about the same time.
+template <int NACC, int J>
+__global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint32_t nrange,
+                                                       uint32_t ntile, uint64_t total,
+                                                       uint64_t off) {
   const int wv = threadIdx.x >> 6;
-  const uint32_t bh = (uint32_t)(wv % WPT) * 8 * NACC;  // the wave's antenna offset
-  __shared__ float2 sP[kMaxUsers * 64];
-  const uint32_t wg = xcd_linear(blockIdx.x, gridDim.x);
-  const uint32_t ab = wg % nab, g = wg / nab;
-  const uint32_t U = a.U, B = a.B, N = a.N, sg = a.sg;
-  const uint32_t b0 = ab * 64;
   const int l = threadIdx.x & 63, i16 = l & 15, q = l >> 4;
-  const int up = q >> 1, p = q & 1, h = i16 & 1;
+  const uint32_t wg = xcd_linear(blockIdx.x, gridDim.x);
+  const uint32_t ab = wg / nrange, rg = wg % nrange;
+  const uint32_t U = a.U, B = a.B, N = a.N, sg = a.sg;
+  const uint32_t b0 = (ab * 4 + wv) * 8 * NACC;
+  if (b0 >= B) return;  // no barriers below
+  const bool h = i16 & 1;
   const uint32_t ncol = sg * a.S;
-  // B operands of tile t: column n of the tile (past the group: its last
-  // column, results dropped), K index q = 2 * (user within the step) + part
-  auto load_x = [&](uint32_t t, float (&bv)[NKS]) {
-    const uint32_t n = min(16 * t + i16, ncol - 1);
-    const uint32_t s = n / sg, k = g * sg + (n - s * sg);
-    const float2* xcol = a.ue + (uint64_t)s * a.ue_sym + k;
+  uint64_t w = total * rg / nrange;
+  const uint64_t w1 = total * (rg + 1) / nrange;
+  if (w >= w1) return;
+  uint32_t g = (uint32_t)(w / ntile), t = (uint32_t)(w % ntile);
+  constexpr int PD = 2;
+  float p1[J][NACC], p2[J][NACC];
+  // antennas past B and users past U clamped (dropped rows, zero symbols)
+  auto load_p = [&](uint32_t gg) {
+    const char* P = reinterpret_cast<const char*>(a.prec + (uint64_t)gg * U * B);
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const uint32_t u = 2 * ks + up;
-      const float2 x = u < U ? xcol[(uint64_t)u * N] : make_float2(0.f, 0.f);
-      bv[ks] = p ? x.y : x.x;
+    for (int j = 0; j < J; ++j) {
+      const uint32_t row = min(4u * j + q, U - 1) * B;
+#pragma unroll
+      for (int m = 0; m < NACC; ++m) {
+        const uint32_t e = row + min(b0 + 8u * m + (i16 >> 1), B - 1);
+        const float2 v = *reinterpret_cast<const float2*>(P + e * 8u);
+        p1[j][m] = h ? v.y : v.x;
+        p2[j][m] = h ? v.x : -v.y;
+      }
     }
   };
-  const float2* P = a.prec + (uint64_t)g * U * B;
-  for (uint32_t e = threadIdx.x; e < U * 64; e += 256) {
-    const uint32_t u = e / 64, bb = e % 64;
-    sP[e] = b0 + bb < B ? P[(uint64_t)u * B + b0 + bb] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  // A operand of row 2r + h and K (user, part p): Re P when h == p, else
-  // -Im P (h = 0) or Im P (h = 1)
-  const bool take_re = h == p;
-  const float sgn = h ? 1.f : -1.f;
-  for (uint32_t t = wv / WPT; t < ntile; t += 4 / WPT) {
-    float bv[NKS];
-    load_x(t, bv);
+  // user symbols of column 16 t + i16 (past the group: its last column, whose
+  // results are dropped), users 4 j + q
+  auto load_x = [&](uint32_t gg, uint32_t tt, float2 (&x)[J]) {
+    const uint32_t n = min(16 * tt + i16, ncol - 1), s = n / sg;
+    const float2* xcol = a.ue + (uint64_t)s * a.ue_sym + (uint64_t)gg * sg + (n - s * sg);
+#pragma unroll
+    for (int j = 0; j < J; ++j) x[j] = xcol[(uint64_t)min(4u * j + q, U - 1) * N];
+  };
+  auto mask_x = [&](float2 (&x)[J]) {
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      if (4u * j + q >= U) x[j] = make_float2(0.f, 0.f);
+  };
+  // the ring's load cursor: PD - 1 tiles ahead, held at the range's last tile
+  uint64_t wl = w;
+  uint32_t gl = g, tl = t;
+  auto fetch = [&](float2 (&x)[J]) {
+    load_x(gl, tl, x);
+    if (wl + 1 < w1) {
+      ++wl;
+      if (++tl == ntile) tl = 0, ++gl;
+    }
+  };
+  float2 x[PD][J];
+#pragma unroll
+  for (int d = 0; d < PD - 1; ++d) fetch(x[d]);
+  load_p(g);
+  // the finished tile: its outputs are stored among the next tile's products
+  v4f done[NACC];
+  float2* O = nullptr;
+  uint64_t row = a.row;
+  auto store = [&](int i) {
+    const int m = i / 2, r = i % 2;
+    const uint32_t b = b0 + 8 * m + 2 * q + r;
+    if (O && b < B) O[(uint64_t)(8 * m + r) * row] = make_float2(done[m][2 * r], done[m][2 * r + 1]);
+  };
+  auto step = [&](float2 (&xc)[J], float2 (&xl)[J]) {
+    fetch(xl);
+    if (4 * J > U) mask_x(xc);
     v4f acc[NACC];
 #pragma unroll
     for (int m = 0; m < NACC; ++m) acc[m] = v4f{0.f, 0.f, 0.f, 0.f};
+    __asm__("" : "+s"(row));
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      if (2 * ks >= (int)U) break;  // uniform
-      const uint32_t u = min(2 * ks + up, U - 1);  // u >= U: bv = 0 makes it inert
-      const float2* prow = sP + u * 64 + bh + (i16 >> 1);
+    for (int j = 0; j < J; ++j) {
 #pragma unroll
-      for (int m = 0; m < NACC; ++m) {
-        const float2 pv = prow[8 * m];
-        const float av = take_re ? pv.x : sgn * pv.y;
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[ks], acc[m], 0, 0, 0);
-      }
+      for (int m = 0; m < NACC; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(p1[j][m], xc[j].x, acc[m], 0, 0, 0);
+#pragma unroll
+      for (int m = 0; m < NACC; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(p2[j][m], xc[j].y, acc[m], 0, 0, 0);
+#pragma unroll
+      for (int i = 2 * NACC * j / J; i < 2 * NACC * (j + 1) / J; ++i) store(i);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    const uint32_t n_raw = 16 * t + i16;
-    if (n_raw < ncol) {
-      const uint32_t s = n_raw / sg, k = g * sg + (n_raw - s * sg);
-      const uint64_t col = ((uint64_t)k + a.bs_start + a.row / 2) % a.row;
-      float2* O = a.out + (uint64_t)s * a.out_sym + col;
 #pragma unroll
-      for (int m = 0; m < NACC; ++m) {
-        const uint32_t b = b0 + bh + 8 * m + 2 * q;
-        if (b < B) O[(uint64_t)b * a.row] = make_float2(acc[m][0], acc[m][1]);
-        if (b + 1 < B) O[(uint64_t)(b + 1) * a.row] = make_float2(acc[m][2], acc[m][3]);
-      }
+    for (int m = 0; m < NACC; ++m) done[m] = acc[m];
+    const uint32_t n = 16 * t + i16, s = n / sg;
+    // off = (bs_start + row / 2) % row
+    uint64_t col = (uint64_t)g * sg + (n - s * sg) + off;
+    if (N <= row)
+      col -= col >= row ? row : 0;
+    else
+      col %= row;
+    O = n < ncol ? a.out + (uint64_t)s * a.out_sym + col + (uint64_t)(b0 + 2 * q) * row : nullptr;
+    if (++t == ntile) {
+      t = 0;
+      ++g;
+      if (w + 1 < w1) load_p(g);
     }
+    return ++w == w1;
+  };
+  for (;;) {
+    bool end = false;
+#pragma unroll
+    for (int d = 0; d < PD; ++d)
+      if (!end) end = step(x[d], x[(d + PD - 1) % PD]);
+    if (end) break;
   }
+#pragma unroll
+  for (int i = 0; i < 2 * NACC; ++i) store(i);
+}
+
+template <int NACC, int J>
+hipError_t precode_run(const PrecodeArgs& a, uint64_t G, uint32_t ntile, hipStream_t st,
+                       const char** why) {
+  const uint64_t total = G * ntile;
+  const uint64_t nab = ((uint64_t)a.B + 32 * NACC - 1) / (32 * NACC);
+  // two workgroups a CU: ranges as long as that leaves them
+  const uint64_t nrange = std::min(total, std::max<uint64_t>(1, 512 / nab));
+  if (nab * nrange > 0x7fffffffull) {
+    *why = "grid too large";
+    return hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL((precode_mfma<NACC, J>), dim3((uint32_t)(nab * nrange)), dim3(256), 0, st, a,
+                     (uint32_t)nrange, ntile, total, (a.bs_start + a.row / 2) % a.row);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -121,32 +188,22 @@ hipError_t launch_precode(const PrecodeArgs& a, hipStream_t st, const char** why
     return hipErrorInvalidValue;
   }
   const uint64_t G = a.N / a.sg;  // full groups only, as the reference
-  const uint64_t nab = (a.B + 63) / 64;
-  const uint64_t ntile = ((uint64_t)a.sg * a.S + 15) / 16;
-  if ((uint64_t)a.sg * a.S > 0xffffffffull || G * nab > 0xffffffffull) {
+  if ((uint64_t)a.sg * a.S > 0xfffffff0ull) {
     *why = "grid too large";
     return hipErrorInvalidValue;
   }
-  const dim3 grid((uint32_t)(G * nab)), block(256);
-  // 32 antennas per wave (fewer registers, one more wave per SIMD at 32
-  // users: 3% faster at 256x32); MEGA_PREC_ACC=8 selects 64
-  const bool half = tune(kPrecAcc) != 8;
-#define MEGA_PREC(UM)                                                                       \
-  if (half)                                                                                  \
-    hipLaunchKernelGGL((precode_mfma<UM, 4>), grid, block, 0, st, a, (uint32_t)nab,          \
-                       (uint32_t)ntile);                                                     \
-  else                                                                                       \
-    hipLaunchKernelGGL((precode_mfma<UM, 8>), grid, block, 0, st, a, (uint32_t)nab,          \
-                       (uint32_t)ntile);
+  const uint32_t ntile = (uint32_t)(((uint64_t)a.sg * a.S + 15) / 16);
+#define MEGA_PREC(J)                                                     \
+  return a.B <= 64 ? precode_run<2, J>(a, G, ntile, st, why) \
+                   : precode_run<(J > 8 ? 2 : 4), J>(a, G, ntile, st, why);
   if (a.U <= 16) {
-    MEGA_PREC(16)
+    MEGA_PREC(4)
   } else if (a.U <= 32) {
-    MEGA_PREC(32)
+    MEGA_PREC(8)
   } else {
-    MEGA_PREC(64)
+    MEGA_PREC(16)
   }
 #undef MEGA_PREC
-  return hipGetLastError();
 }
 
 }  // namespace detail

@@ -33,7 +33,6 @@ constexpr TuneSpec kSpecs[kTuneCount] = {
     {"MEGA_EQ_XREG", 0, 0, 1},    // mixed equalize: 1 forces streamed W
     {"MEGA_EQ_XT", 0, 1, 2},      // mixed equalize: column tiles per wave
     {"MEGA_EQ_XKS", 0, 1, 4},     // mixed equalize: waves per unit (antenna split)
-    {"MEGA_PREC_ACC", 0, 8, 8},   // precode: 8 = 64 antennas per wave
     {"MEGA_DET_PF", 1, 0, 1},     // fused detect: next-tile y prefetch
     {"MEGA_EQ_WTC", 0, 1, 1 << 20},  // FP32 wide form: column tiles per workgroup
     {"MEGA_ZF_NTH", 0, 256, 512},   // FP32 ZF threads per group: 512 (17-32 users), 256 (33-64)

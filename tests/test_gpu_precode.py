@@ -65,3 +65,51 @@ def test_precode_matches_oracle(B, U, N, sg, row, start, S):
     if N < sg:
         assert (got == SENT).all()
 
+
+
+@pytest.mark.parametrize("B,U,N,sg,row,start,S", [
+    (97, 40, 500, 8, 512, 6, 14),    # 33-64 users, 434 tiles over two antenna blocks' ranges
+    (300, 20, 333, 7, 512, 300, 3),  # the shift wraps round the row; three antenna blocks
+    (200, 32, 1637, 12, 2048, 205, 14),  # ranges that cross groups at every place of a tile
+    (1, 1, 40, 3, 64, 1, 1),
+])
+def test_precode_ranges_match_fp64(B, U, N, sg, row, start, S):
+    """The register kernel's ranges, antenna blocks and user steps: FP32 sums
+    of U products, so within U * 2^-23 of the sum of magnitudes; untouched
+    columns stay."""
+    print(f"case: precode ranges B={B} U={U} N={N} sg={sg} S={S}", flush=True)
+    t = torch()
+    rng = np.random.default_rng(B + U + N)
+    G, full = -(-N // sg), N // sg
+    P = (rng.standard_normal((G, U, B)) + 1j * rng.standard_normal((G, U, B))).astype(np.complex64)
+    ue = (rng.standard_normal((S, U, N)) + 1j * rng.standard_normal((S, U, N))).astype(np.complex64)
+    out = t.from_numpy(np.full((S, B, row), SENT, np.complex64)).to("cuda:0")
+    m.precode(dev_c64(P.reshape(-1)), dev_c64(ue.reshape(-1)), out, num_bs=B, num_ue=U, num_sc=N,
+              sc_group=sg, bs_stride=row, bs_start=start, num_syms=S)
+    got = host_c64(out).reshape(S, B, row)
+    exp = np.full((S, B, row), SENT, np.complex128)
+    mag = np.zeros((S, B, row))
+    for g in range(full):
+        k = np.arange(g * sg, (g + 1) * sg)
+        col = (k + start + row // 2) % row
+        exp[:, :, col] = np.einsum("ub,suk->sbk", P[g].astype(np.complex128), ue[:, :, k])
+        mag[:, :, col] = np.einsum("ub,suk->sbk", np.abs(P[g]), np.abs(ue[:, :, k]))
+    untouched = mag == 0
+    assert np.array_equal(got[untouched], exp[untouched].astype(np.complex64))
+    assert (np.abs(got - exp) <= 4 * U * 2.0 ** -23 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("U,B,G", [(1, 1, 3), (32, 256, 5), (64, 256, 2), (128, 300, 2), (100, 1, 4),
+                                   (17000, 2, 1)])
+def test_precoder_normalisation_shapes(U, B, G):
+    """One LDS tile, several tiles and none: P = W^T / max|W| within the two
+    roundings of 1 / max and the product."""
+    print(f"case: precoder normalisation U={U} B={B} G={G}", flush=True)
+    t = torch()
+    rng = np.random.default_rng(U + B)
+    W = (rng.standard_normal((G, B, U)) + 1j * rng.standard_normal((G, B, U))).astype(np.complex64)
+    P = t.zeros(G, U, B, dtype=t.complex64, device="cuda:0")
+    m.Beamform.beamform_downlink(dev_c64(W.reshape(-1)), P, U, B, G)
+    got = host_c64(P).reshape(G, U, B)
+    exp = (W / np.abs(W.astype(np.complex128)).max((1, 2), keepdims=True)).swapaxes(1, 2)
+    assert np.abs(got - exp).max() < 4 * 2.0 ** -23
