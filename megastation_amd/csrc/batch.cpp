@@ -30,10 +30,12 @@ struct ZfClass {
 
 struct EqPlanChoice {
   EqKind kind = EqKind::Stream;
-  uint32_t MT = 4, KS = 0, waves_per_cu = 12;
+  uint32_t MT = 4, KS = 0, waves_per_cu = 12, chunks = 1;
   std::string str() const {
     std::ostringstream o;
-    if (kind == EqKind::Stream)
+    if (kind == EqKind::Wide)
+      o << "wide MT=" << MT << " KS=" << KS << " chunks=" << chunks;
+    else if (kind == EqKind::Stream)
       o << "stream MT=" << MT << " waves/CU=" << waves_per_cu;
     else
       o << "reg MT=" << MT << " KS=" << KS;
@@ -46,6 +48,11 @@ struct EqPlanChoice {
     }
     if (std::sscanf(s.c_str(), "reg MT=%u KS=%u", &c.MT, &c.KS) == 2) {
       c.kind = EqKind::Reg;
+      return true;
+    }
+    if (std::sscanf(s.c_str(), "wide MT=%u KS=%u chunks=%u", &c.MT, &c.KS, &c.chunks) == 3 &&
+        c.chunks >= 1) {
+      c.kind = EqKind::Wide;
       return true;
     }
     return false;
@@ -70,6 +77,11 @@ uint32_t eq_units(EqParams& p, const EqPlanChoice& c) {
     p.tiles_per_wg = p.col_tiles;
     return p.G * p.col_tiles * p.nmg;
   }
+  if (c.kind == EqKind::Wide) {
+    p.tiles_per_wg = (p.col_tiles + c.chunks - 1) / c.chunks;
+    p.chunks = (p.col_tiles + p.tiles_per_wg - 1) / p.tiles_per_wg;
+    return p.G * p.chunks;
+  }
   p.nmg = (p.U + 8 * c.MT - 1) / (8 * c.MT);
   p.nwk = 1;
   // column tiles of a group split into chunks of about 4 tiles
@@ -78,9 +90,25 @@ uint32_t eq_units(EqParams& p, const EqPlanChoice& c) {
   return p.G * p.chunks * p.nmg;
 }
 
+// 16-user tiles of a class (the wide form's).
+uint32_t user_tiles(uint32_t U) { return U <= 16 ? 1 : U <= 32 ? 2 : 4; }
+
 std::vector<EqPlanChoice> eq_candidates(uint32_t B, uint32_t maxU) {
   std::vector<EqPlanChoice> v;
-  if (B % 32 == 0) {
+  // The wide form up to 256 antennas, W_g once per chunk of a group's column
+  // tiles: one or two chunks where the batch fills the chip, five for short
+  // batches. Beyond, streamed W (256 x 64, 1667 groups: 385 us against 516
+  // streamed; 128 x 32, 1655 groups: 110 against 145).
+  if (B % 32 == 0 && B > 32 && B <= 256) {
+    for (uint32_t n : {1u, 2u, 5u}) {
+      EqPlanChoice c;
+      c.kind = EqKind::Wide;
+      c.MT = user_tiles(maxU);
+      c.KS = B <= 128 ? 4 : 8;
+      c.chunks = n;
+      v.push_back(c);
+    }
+  } else if (B % 32 == 0) {
     for (uint32_t MT : {1u, 2u, 4u}) {
       if (MT > 1 && 8 * (MT / 2) >= maxU) continue;  // a smaller tile already covers all users
       for (uint32_t w : {8u, 12u, 16u}) {
@@ -300,9 +328,9 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
     b->zf.push_back(z);
   }
   {
-    std::map<uint32_t, EqClass> byB;
+    std::map<std::pair<uint32_t, uint32_t>, EqClass> byB;
     for (uint32_t i = 0; i < num_cells; ++i) {
-      EqClass& c = byB[b->eqp[i].B];
+      EqClass& c = byB[{b->eqp[i].B, user_tiles(b->eqp[i].U)}];
       c.B = b->eqp[i].B;
       c.cells.push_back(i);
     }
@@ -419,7 +447,6 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
       L.kind = q.plan.kind;
       L.MT = q.plan.MT;
       L.KS = q.plan.KS;
-      L.nch = (q.B == 64 || q.B == 128 || q.B == 256) ? q.B / 8 : 0;
       L.cells = reinterpret_cast<const BatchCell*>(at(eq_cells_off[k]));
       L.ncells = (uint32_t)q.cells.size();
       L.prefix = reinterpret_cast<const uint32_t*>(at(eq_prefix_off[k]));
@@ -432,7 +459,8 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
         total += eq_units(p, q.plan);
       }
       const uint32_t wgs = (total + 3) / 4;
-      L.blocks = q.plan.kind == EqKind::Stream
+      L.blocks = q.plan.kind == EqKind::Wide ? total
+                 : q.plan.kind == EqKind::Stream
                      ? std::min<uint32_t>(wgs, kCUs * q.plan.waves_per_cu / 4)
                      : wgs;
       b->eq_launch.push_back(L);
@@ -455,7 +483,13 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
       return bail(MEGA_ERR_UNSUPPORTED, "no equalize plan for B=" + std::to_string(q.B));
     q.plan = cands[0];
     auto it = cache.find(q.key);
-    if (it != cache.end() && EqPlanChoice::parse(it->second, q.plan)) tune[k] = false;
+    EqPlanChoice saved;
+    if (it != cache.end() && EqPlanChoice::parse(it->second, saved) &&
+        (saved.kind != EqKind::Wide ||
+         (q.B <= 256 && saved.MT == user_tiles(maxU) && saved.KS == (q.B <= 128 ? 4u : 8u)))) {
+      q.plan = saved;
+      tune[k] = false;
+    }
   }
   if ((e = build()) != hipSuccess) return hip_bail(e, "batch tables");
   if ((e = run_launches(b, b->stream, false)) != hipSuccess) return hip_bail(e, "batch warm-up");

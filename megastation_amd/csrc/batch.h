@@ -27,15 +27,15 @@ struct ZfClassLaunch {
   uint32_t ncells;
 };
 
-enum class EqKind : uint32_t { Stream = 0, Reg = 1 };
+enum class EqKind : uint32_t { Stream = 0, Reg = 1, Wide = 2 };
 
 struct EqClassLaunch {
   EqKind kind;
-  uint32_t MT, KS, nch;    // tile plan (nch: stream chunk count, 0 = runtime)
+  uint32_t MT, KS;         // tile plan
   uint32_t blocks;         // grid (persistent for Stream)
   const BatchCell* cells;
   uint32_t ncells;
-  const uint32_t* prefix;   // Reg: device, ncells + 1 unit prefix sums
+  const uint32_t* prefix;   // Reg, Wide: device, ncells + 1 unit prefix sums
   const uint32_t* xprefix;  // Stream: [8][ncells + 1] per-XCD queue prefix sums
   const uint32_t* xbase;    // Stream: [8][ncells] first unit of each cell's part
   uint32_t* counters;       // Stream: the 8 queue counters

@@ -5,14 +5,18 @@
 //   ZF classes  - users rounded up to 16-row tiles (UT = 1, 2, 4); one
 //                 workgroup per (cell, group), the cell found from a prefix
 //                 table of group counts (zf_core.h does the group's work);
-//   EQ classes  - antenna count and the tile plan the autotuner picked for
-//                 it (streamed W with MT 8-user M tiles per wave, or W held
-//                 in registers); a persistent grid whose waves take units
-//                 (cell, group, column tile, user group) from a work counter
-//                 until it runs out, longest cells first.
-// The modulation order is a per-cell runtime value (the demod epilogue
-// switches on it), so it does not split classes.
+//   EQ classes  - antenna count, users rounded up to 16-row tiles, and the
+//                 tile plan the autotuner picked for them: the wide form's
+//                 units (eq_wide.h), W held in one wave's registers, or, past
+//                 256 antennas, streamed W on a persistent grid whose waves
+//                 take units from a work counter, longest cells first.
+// The modulation order is a per-cell value: a unit switches on it once, to the
+// code with that order's demod, so it does not split classes. (One switch per
+// stored output kept the compiler from scheduling loads and products across
+// outputs: the streamed form took 84 us a 256 x 64 slot with the order known
+// and 130 with it looked up.)
 #include "batch.h"
+#include "eq_wide.h"
 #include "zf_core.h"
 
 namespace mega {
@@ -56,15 +60,28 @@ __global__ __launch_bounds__(cells_threads<UT>(), UT == 2 ? 3 : 1) void zf_cells
   if (threadIdx.x == 0 && cell.info) cell.info[g] = fail;
 }
 
+// f with the cell's modulation order as a compile-time value.
+template <typename F>
+__device__ __forceinline__ void with_order(uint32_t q, F&& f) {
+  switch (q) {
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
+  }
+}
+
 // Equalize unit u of a cell (streamed W): u = ((g * col_tiles) + t) * nmg + mg.
-template <int MT, int KC, int R, int NCH>
+template <int MT, int KC, int R>
 __device__ __forceinline__ void eq_cell_unit(const BatchCell& cell, uint32_t u) {
   const EqParams& p = cell.eq;
   const uint32_t mg = u % p.nmg;
   const uint32_t t = (u / p.nmg) % p.col_tiles;
   const uint32_t g = u / p.nmg / p.col_tiles;
   if (16 * t >= min(p.sg, p.N - g * p.sg) * p.S) return;  // past a partial group
-  eq_unit_stream<MT, KC, R, NCH, 0>(p, 0, g, t, mg);  // runtime-Q epilogue
+  with_order(p.Q, [&](auto q) {
+    eq_unit_stream<MT, KC, R, 0, decltype(q)::value>(p, 0, g, t, mg);
+  });
 }
 
 // Persistent streamed-W equalize over a class. The units are split into 8
@@ -74,7 +91,7 @@ __device__ __forceinline__ void eq_cell_unit(const BatchCell& cell, uint32_t u) 
 // dealt to XCDs round-robin, so blockIdx % 8) and then helps the others; it
 // takes one unit per vector atomic on the queue's counter (lane 0, then
 // broadcast) and exits when every queue is past its end.
-template <int MT, int NCH>
+template <int MT>
 __global__ __launch_bounds__(256) void eq_cells_stream(const BatchCell* cells,
                                                        const uint32_t* xprefix,
                                                        const uint32_t* xbase, uint32_t ncells,
@@ -90,7 +107,7 @@ __global__ __launch_bounds__(256) void eq_cells_stream(const BatchCell* cells,
       i = __shfl(i, 0, 64);
       if (i >= end) break;
       const uint32_t c = find_cell(px, ncells, i);
-      eq_cell_unit<MT, 2, 4, NCH>(cells[c], xbase[x * ncells + c] + (i - px[c]));
+      eq_cell_unit<MT, 2, 4>(cells[c], xbase[x * ncells + c] + (i - px[c]));
     }
   }
 }
@@ -120,7 +137,28 @@ __global__ __launch_bounds__(256) void eq_cells_reg(const BatchCell* cells,
   eq_load_tile<KS>(p, 0, g, 0, t0, ynext);
   WRegs<MT, KS> ws;
   ws.load(W, p.U, p.U, p.B, mg, 0);
-  eq_tiles<MT, KS, 0>(p, ws, 0, g, mg, 0, t0, t1, nullptr, ynext);  // runtime Q
+  with_order(p.Q, [&](auto q) {
+    eq_tiles<MT, KS, decltype(q)::value>(p, ws, 0, g, mg, 0, t0, t1, nullptr, ynext);
+  });
+}
+
+// Wide form: one eight-wave workgroup per (cell, group, chunk of column tiles).
+template <int MT, int KS>
+__global__ __launch_bounds__(512, eq_wide_waves(MT, 8)) void eq_cells_wide(const BatchCell* cells,
+                                                                            const uint32_t* prefix,
+                                                                            uint32_t ncells) {
+  __shared__ EqWideRed<MT, 8> red;
+  const uint32_t unit = xcd_linear(blockIdx.x, gridDim.x);
+  const uint32_t c = find_cell(prefix, ncells, unit);
+  const EqParams p = cells[c].eq;
+  const uint32_t u = unit - prefix[c];
+  const uint32_t g = u / p.chunks;
+  const uint32_t t0 = (u - g * p.chunks) * p.tiles_per_wg;
+  const uint32_t t1 = min(t0 + p.tiles_per_wg, (min(p.sg, p.N - g * p.sg) * p.S + 15) / 16);
+  if (t0 >= t1) return;  // past a partial group: uniform
+  with_order(p.Q, [&](auto q) {
+    eq_wide_unit<MT, KS, 8, decltype(q)::value>(p, 0, g, t0, t1, red);
+  });
 }
 
 __global__ void reset_counters(uint32_t* c, uint32_t n) {
@@ -152,22 +190,6 @@ hipError_t launch_zf_ut(const ZfClassLaunch& L, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int MT>
-hipError_t launch_stream_mt(const EqClassLaunch& L, hipStream_t st) {
-  const dim3 grid(L.blocks), block(256);
-#define MEGA_EQ_CELLS(NCH)                                                                  \
-  hipLaunchKernelGGL((eq_cells_stream<MT, NCH>), grid, block, 0, st, L.cells, L.xprefix, \
-                     L.xbase, L.ncells, L.counters)
-  switch (L.nch) {
-    case 8: MEGA_EQ_CELLS(8); break;
-    case 16: MEGA_EQ_CELLS(16); break;
-    case 32: MEGA_EQ_CELLS(32); break;
-    default: MEGA_EQ_CELLS(0); break;
-  }
-#undef MEGA_EQ_CELLS
-  return hipGetLastError();
-}
-
 }  // namespace
 
 hipError_t prepare_zf_class(const ZfClassLaunch& L) {
@@ -192,12 +214,34 @@ hipError_t launch_zf_class(const ZfClassLaunch& L, hipStream_t st) {
 hipError_t launch_eq_class(const EqClassLaunch& L, hipStream_t st) {
   if (L.blocks == 0) return hipSuccess;
   if (L.kind == EqKind::Stream) {
+    const dim3 grid(L.blocks), block(256);
+#define MEGA_EQ_CELLS(MT)                                                              \
+  hipLaunchKernelGGL((eq_cells_stream<MT>), grid, block, 0, st, L.cells, L.xprefix, \
+                     L.xbase, L.ncells, L.counters)
     switch (L.MT) {
-      case 1: return launch_stream_mt<1>(L, st);
-      case 2: return launch_stream_mt<2>(L, st);
-      case 4: return launch_stream_mt<4>(L, st);
+      case 1: MEGA_EQ_CELLS(1); break;
+      case 2: MEGA_EQ_CELLS(2); break;
+      case 4: MEGA_EQ_CELLS(4); break;
       default: return hipErrorInvalidValue;
     }
+#undef MEGA_EQ_CELLS
+    return hipGetLastError();
+  }
+  if (L.kind == EqKind::Wide) {
+    const dim3 grid(L.blocks), block(512);
+#define MEGA_EQ_CELLS(MT, KS) \
+  hipLaunchKernelGGL((eq_cells_wide<MT, KS>), grid, block, 0, st, L.cells, L.prefix, L.ncells)
+    switch (L.MT * 100 + L.KS) {
+      case 104: MEGA_EQ_CELLS(1, 4); break;
+      case 108: MEGA_EQ_CELLS(1, 8); break;
+      case 204: MEGA_EQ_CELLS(2, 4); break;
+      case 208: MEGA_EQ_CELLS(2, 8); break;
+      case 404: MEGA_EQ_CELLS(4, 4); break;
+      case 408: MEGA_EQ_CELLS(4, 8); break;
+      default: return hipErrorInvalidValue;
+    }
+#undef MEGA_EQ_CELLS
+    return hipGetLastError();
   }
   const dim3 grid(L.blocks), block(256);
   switch (L.MT * 100 + L.KS) {
