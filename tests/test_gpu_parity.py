@@ -122,6 +122,26 @@ def test_zf_thread_counts_are_bit_identical(U, B, G, tuning):
     assert (np.linalg.norm(w - ref, axis=1) / np.linalg.norm(ref, axis=1)).max() < 1e-4
 
 
+@pytest.mark.parametrize("U,B,G", [(33, 67, 5), (40, 600, 7), (48, 260, 4), (49, 70, 3)])
+def test_zf_padded_user_tiles_are_bit_identical(U, B, G, tuning):
+    """Sixteen waves leave out the tiles of users past U and add the Gram's
+    chunks in rounds of four through LDS (600 antennas: three rounds, the last
+    partial); four waves compute every tile. Same bits, also in place."""
+    print(f"case: zf padded tiles U={U} B={B} G={G}", flush=True)
+    t = torch()
+    rng = np.random.Generator(np.random.Philox(U * 11 + B))
+    a = np.conj(synth.channel_iid(rng, G, B, U)).astype(np.complex64)
+    outs = []
+    for nth in (256, 0):
+        tuning(MEGA_ZF_NTH=nth)
+        d = dev_c64(a.reshape(-1))
+        m.zf(d, d, B, U, G)
+        _sync()
+        outs.append(host_c64(d).view(np.uint32))
+    assert np.array_equal(outs[0], outs[1])
+    assert np.abs(outs[0].view(np.complex64)).max() > 0
+
+
 @pytest.mark.parametrize("U,B", [(8, 32), (100, 200)])
 def test_zf_in_place_and_failed_groups(U, B):
     print(f"case: zf in place with rank-deficient groups U={U} B={B}", flush=True)
