@@ -153,11 +153,8 @@ __global__ __launch_bounds__(512, eq_wide_waves(MT, 8)) void eq_cells_wide(const
   const EqParams p = cells[c].eq;
   const uint32_t u = unit - prefix[c];
   const uint32_t g = u / p.chunks;
-  const uint32_t t0 = (u - g * p.chunks) * p.tiles_per_wg;
-  const uint32_t t1 = min(t0 + p.tiles_per_wg, (min(p.sg, p.N - g * p.sg) * p.S + 15) / 16);
-  if (t0 >= t1) return;  // past a partial group: uniform
   with_order(p.Q, [&](auto q) {
-    eq_wide_unit<MT, KS, 8, decltype(q)::value>(p, 0, g, t0, t1, red);
+    eq_wide_unit<MT, KS, 8, decltype(q)::value>(p, 0, g, u - g * p.chunks, p.tiles_per_wg, red);
   });
 }
 

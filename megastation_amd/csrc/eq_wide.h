@@ -42,16 +42,19 @@ constexpr int eq_wide_waves(int MT, int NW) { return NW == 8 && MT <= 2 ? 4 : 2;
 template <int MT, int NW>
 using EqWideRed = float[2][NW][MT][2][4][64];
 
-// Column tiles [t0, t1) of group g of a slot, by one workgroup of NW waves.
+// Chunk c of tc column tiles of group g of a slot, by one workgroup of NW waves.
 template <int MT, int KS, int NW, int Q>
 __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, uint32_t g,
-                                             uint32_t t0, uint32_t t1, EqWideRed<MT, NW>& red) {
+                                             uint32_t c, uint32_t tc, EqWideRed<MT, NW>& red) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i16 = lane & 15, q4 = lane >> 4;
   const uint32_t U = p.U, B = p.B, N = p.N;
   const uint32_t k0 = g * p.sg;
   const uint32_t nk = min(p.sg, N - k0);
   const uint32_t ncol = nk * p.S;
+  const uint32_t t0 = c * tc;
+  const uint32_t t1 = min(t0 + tc, (ncol + 15) / 16);
+  if (t0 >= t1) return;  // a chunk past a partial group: uniform
 
   // ---- this wave's W slice: Wr, Wi per (user tile, step); Wr + Wi is formed
   // at each use (one add per MFMA triple saves a third of the slice's
@@ -123,16 +126,47 @@ __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, u
     v4f k1[MT], k2[MT], k3[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) k1[m] = k2[m] = k3[m] = v4f{0.f, 0.f, 0.f, 0.f};
+    // An FP32 MFMA and the vector ALU exclude each other, and a switch between
+    // them costs 6 to 14 cycles: up to two user tiles the operands of each of two
+    // bursts are formed ahead of it (42.7 us a 256 x 32 slot against 44.1 with
+    // the sums beside the products). Four tiles have no registers for it.
+    if constexpr (MT <= 2) {
+      float ws[MT][KS], yd[KS], yp[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const float yr = ycur[s].x;
-      const float yd = ycur[s].y - ycur[s].x;
-      const float yp = ycur[s].x + ycur[s].y;
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        k1[m] = mfma4(wre[m][s] + wim[m][s], yr, k1[m]);
-        k2[m] = mfma4(wre[m][s], yd, k2[m]);
-        k3[m] = mfma4(wim[m][s], yp, k3[m]);
+        for (int s = 0; s < KS; ++s) ws[m][s] = wre[m][s] + wim[m][s];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) k1[m] = mfma4(ws[m][s], ycur[s].x, k1[m]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        yd[s] = ycur[s].y - ycur[s].x;
+        yp[s] = ycur[s].x + ycur[s].y;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          k2[m] = mfma4(wre[m][s], yd[s], k2[m]);
+          k3[m] = mfma4(wim[m][s], yp[s], k3[m]);
+        }
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const float yr = ycur[s].x;
+        const float yd = ycur[s].y - ycur[s].x;
+        const float yp = ycur[s].x + ycur[s].y;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          k1[m] = mfma4(wre[m][s] + wim[m][s], yr, k1[m]);
+          k2[m] = mfma4(wre[m][s], yd, k2[m]);
+          k3[m] = mfma4(wim[m][s], yp, k3[m]);
+        }
       }
     }
 #pragma unroll

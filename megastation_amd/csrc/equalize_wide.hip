@@ -17,10 +17,7 @@ __global__ __launch_bounds__(64 * NW, eq_wide_waves(MT, NW)) void equalize_wide(
   const uint32_t c = unit % chunks;
   const uint32_t rest = unit / chunks;
   const uint32_t g = rest % p.G, slot = rest / p.G;
-  const uint32_t t0 = c * tc;
-  const uint32_t t1 = min(t0 + tc, (min(p.sg, p.N - g * p.sg) * p.S + 15) / 16);
-  if (t0 >= t1) return;  // a chunk past a partial group: uniform
-  eq_wide_unit<MT, KS, NW, Q>(p, slot, g, t0, t1, red);
+  eq_wide_unit<MT, KS, NW, Q>(p, slot, g, c, tc, red);
 }
 
 // Persistent form of the same arithmetic: P workgroups, workgroup i sweeping

@@ -94,6 +94,55 @@ def test_batch_matches_single_cell_paths_and_oracle(tmp_path):
     b2.close()
 
 
+WIDE_CELLS = [  # every wide tile plan: 1, 2 and 4 user tiles, 64-128 and 160-256 antennas
+    (16, 96, 204, 12, 2, "standalone"),
+    (20, 64, 100, 16, 4, "ldpc"),
+    (33, 96, 77, 8, 6, "standalone"),
+    (8, 160, 150, 16, 8, "standalone"),
+    (24, 224, 60, 12, 4, "standalone"),
+    (50, 160, 41, 12, 8, "standalone"),
+]
+
+
+def test_batch_wide_plans_agree_for_every_chunk_count(tmp_path, monkeypatch):
+    """The wide units' results do not depend on how a group's column tiles are
+    cut into chunks (1, 2 or 5, forced through the plan file), and match FP64."""
+    print("case: batch wide plans", flush=True)
+    t = torch()
+    monkeypatch.setitem(globals(), "CELLS", WIDE_CELLS)
+    cells = _make_cells(seed=5, S=5)
+    path = tmp_path / "tune.txt"
+    m.Batch(cells, tune_path=str(path)).close()
+    saved = [line.split("\t") for line in path.read_text().splitlines()]
+    outs = []
+    for n in (1, 2, 5):
+        with open(path, "w") as f:
+            for key, _ in saved:
+                B = int(key.split(";")[0][2:])
+                U = max(int(c.split("x")[0]) for c in key.split(";")[1:])
+                mt = 1 if U <= 16 else 2 if U <= 32 else 4
+                f.write(f"{key}\twide MT={mt} KS={4 if B <= 128 else 8} chunks={n}\n")
+        for c in cells:
+            c["llr"].fill_(SENTINEL)
+            c["xhat"].zero_()
+        b = m.Batch(cells, tune_path=str(path))
+        assert b.plan().count("(cached)") == len(saved)
+        b.run()
+        t.cuda.synchronize()
+        outs.append([(host_u16(c["llr"]).copy(), host_c64(c["xhat"]).copy()) for c in cells])
+        b.close()
+    for other in outs[1:]:
+        for (l0, x0), (l1, x1) in zip(outs[0], other):
+            assert np.array_equal(l0, l1) and np.array_equal(x0, x1)
+    for c, (llr, xh) in zip(cells, outs[0]):
+        U, B, N, sg, Q, S, lay = c["U"], c["B"], c["N"], c["sg"], c["Q"], c["S"], c["layout"]
+        w64, _, _ = oracle.zf(c["slot"].csi, U, B, (N + sg - 1) // sg, "f64")
+        for s in range(S):
+            llr64, x64 = oracle_symbol_f64(w64, c["slot"].y[s], U, B, N, sg, Q, lay)
+            check_symbol(llr.reshape(S, U, lay.ue_stride)[s], xh.reshape(S, U, N)[s], llr64, x64,
+                         N, sg, Q, lay)
+
+
 def test_batch_rejects_bad_cells():
     print("case: batch argument checks", flush=True)
     cells = _make_cells()[:2]
