@@ -74,6 +74,32 @@ def test_decoder_matches_oracle_on_noisy_code_blocks(bg, zc, mb, half):
     print(f"  residual bit errors after 4 iterations: {errs}", flush=True)
 
 
+@pytest.mark.parametrize("bg,zc,mb,half,n_cb", [(1, 288, 46, True, 257), (1, 384, 18, False, 258),
+                                                (2, 320, 42, True, 259), (2, 256, 42, True, 257)])
+def test_more_code_blocks_than_cus_match_oracle(bg, zc, mb, half, n_cb):
+    """More code blocks than the card has CUs: from Zc > 256 on two of them share
+    a workgroup where LDS holds both (the last may be alone). Five different
+    blocks in turn, so that each meets each as its neighbour; bits and the padding
+    after them are equal to the oracle's."""
+    print(f"case: ldpc pairs bg={bg} zc={zc} mb={mb} half={half} n_cb={n_cb}", flush=True)
+    kb = ldpc.KB[bg]
+    rng = np.random.default_rng(zc + mb)
+    info = rng.integers(0, 2, (5, kb * zc)).astype(np.uint8)
+    cws = np.stack([ldpc.encode(b, bg, zc, mb) for b in info])
+    llr = 2 * ((1 - 2.0 * cws) + rng.standard_normal(cws.shape))
+    llr[:, :2 * zc] = 0
+    llr = llr.astype(np.float16 if half else np.float32).astype(np.float32)
+    nv, words = (kb + mb) * zc, (kb * zc + 31) // 32
+    stride = synth.pad64(nv)
+    buf = np.zeros((n_cb, stride), np.float32)
+    turn = np.arange(n_cb) % 5
+    buf[:, :nv] = llr[turn]
+    out = _decode_gpu(buf, bg, zc, mb, 4, half, n_cb, stride, words + 1)
+    ref = ldpc.decode(llr, bg, zc, mb, 4, 0.8125)
+    assert np.array_equal(out[:, :words], ref[turn])
+    assert np.all(out[:, words:] == 0xFFFFFFFF)
+
+
 def test_equalizer_llrs_decode_to_transmitted_bits():
     """64 x 16 cell, 1200 subcarriers, 16-QAM at -4 dB per antenna (about
     13 dB after ZF's array gain; the hard decisions of about 2 % of the coded
