@@ -57,7 +57,7 @@ struct ZfShared {
 // round through LDS; the other waves of a SIMD cover a wave's loads. (A tile a
 // wave, its four chunks one after the other, left six of the 16 waves idle and
 // every chunk's loads in the open: 17.8 us at 48 users x 200 antennas, 11.2
-// now, 24 of those items being the pad's.)
+// now, 16 of its 40 items being the pad's.)
 template <int UT, int NW>
 struct ZfPlan {
   static constexpr int NT = UT * (UT + 1) / 2;
@@ -466,24 +466,55 @@ __device__ __forceinline__ void zf_apply(const float2* A, uint32_t U, uint32_t B
   // A columns of the wave's antenna tiles, the next tile's in flight during
   // this tile's MFMAs (global A: clamped addresses, users past U zeroed)
   float2 abuf[2][KSU];
+  // From global memory a step's four users of an antenna go to a quad of lanes
+  // and change places in registers: the load unit takes a quad's 32 contiguous
+  // bytes at once (17 cycles a load), where in the operand's order (neighbour
+  // lanes in neighbour antennas) every lane costs one (65). So do W's stores,
+  // which is why the antennas are the product's rows: sixteen users of an antenna
+  // a quarter wave. 256 x 32 x 273: 37.1 -> 34.4 us, 256 x 64: 122 -> 117. With
+  // eight user tiles the users stay the rows (as above, 4 % more time).
+  constexpr bool BROW = UT <= 4, QUAD = BROW && !A_LDS;
+  auto prod = [](float av, float gv, v4f acc) {
+    return BROW ? mfma4(av, gv, acc) : mfma4(gv, av, acc);
+  };
   auto fetch_a = [&](uint32_t nb, float2 (&d)[KSU]) {
     if constexpr (A_LDS) {
 #pragma unroll
       for (int s = 0; s < KSU; ++s) d[s] = aval(4 * s + q4, 16 * nb + i16);
     } else {
-      const uint32_t bc = min(16 * min(nb, nb_tiles - 1) + i16, B - 1);
+      const uint32_t bc = min(16 * min(nb, nb_tiles - 1) + (QUAD ? lane / 4 : i16), B - 1);
+      const uint32_t ul = QUAD ? lane % 4 : q4;
 #pragma unroll
-      for (int s = 0; s < KSU; ++s) d[s] = A[min(4u * s + q4, U - 1) + (uint64_t)U * bc];
+      for (int s = 0; s < KSU; ++s) d[s] = A[min(4u * s + ul, U - 1) + (uint64_t)U * bc];
+    }
+  };
+  // the operand lane's entry (antenna i16, user 4 s + q4) of a loaded step
+  auto operand = [&](float2 v, int s) -> float2 {
+    if constexpr (QUAD) {
+      const int from = (4 * i16 + q4) * 4;
+      v.x = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v.x)));
+      v.y = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v.y)));
+    }
+    return 4u * s + q4 < U ? v : make_float2(0.f, 0.f);
+  };
+  auto put = [&](uint32_t u, uint32_t b, float re, float im) {
+    if (u < U) {
+      const float2 v = make_float2(re, im);
+      w[u + (uint64_t)ld_w * b] = v;
+      if (w2) w2[u + (uint64_t)U * b] = v;
+    }
+  };
+  auto store_tile = [&](uint32_t nb, int mi, v4f re, v4f im) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t b = 16 * nb + 4 * q4 + r;
+      if (b < B) put(16 * mi + i16, b, re[r], im[r]);
     }
   };
   auto apply_tile = [&](uint32_t nb, const float2 (&cur)[KSU]) {
-    const uint32_t b = 16 * nb + i16;
     float2 av[KSU];
 #pragma unroll
-    for (int s = 0; s < KSU; ++s) {
-      const bool ok = 4u * s + q4 < U;
-      av[s] = ok ? cur[s] : make_float2(0.f, 0.f);
-    }
+    for (int s = 0; s < KSU; ++s) av[s] = operand(cur[s], s);
     v4f res_r[UT], res_i[UT];
 #pragma unroll
     for (int mi = 0; mi < UT; ++mi) {
@@ -492,27 +523,16 @@ __device__ __forceinline__ void zf_apply(const float2* A, uint32_t U, uint32_t B
       for (int s = 0; s < KSU; ++s) {
         const float2 m = res[(16 * mi + i16) * LDG + 4 * s + q4];
         const float gr = -m.x, gi = -m.y;  // G^-1 = -res
-        wr1 = mfma4(gr, av[s].x, wr1);
-        wr2 = mfma4(-gi, av[s].y, wr2);
-        wi1 = mfma4(gr, av[s].y, wi1);
-        wi2 = mfma4(gi, av[s].x, wi2);
+        wr1 = prod(av[s].x, gr, wr1);
+        wr2 = prod(av[s].y, -gi, wr2);
+        wi1 = prod(av[s].y, gr, wi1);
+        wi2 = prod(av[s].x, gi, wi2);
       }
       res_r[mi] = wr1 + wr2;
       res_i[mi] = wi1 + wi2;
     }
-    if (b < B) {
 #pragma unroll
-      for (int mi = 0; mi < UT; ++mi)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t u = 16 * mi + 4 * q4 + r;
-          if (u < U) {
-            const float2 v = make_float2(res_r[mi][r], res_i[mi][r]);
-            w[u + (uint64_t)ld_w * b] = v;
-            if (w2) w2[u + (uint64_t)U * b] = v;
-          }
-        }
-    }
+    for (int mi = 0; mi < UT; ++mi) store_tile(nb, mi, res_r[mi], res_i[mi]);
   };
   // A wave owns the antenna tiles wave, wave+NW, ...; only its own columns
   // are read (ahead, from global memory) and overwritten, so W may replace A
@@ -522,10 +542,13 @@ __device__ __forceinline__ void zf_apply(const float2* A, uint32_t U, uint32_t B
     // tiles two at a time; the same products and sums as apply_tile
     for (uint32_t nb = wave; nb < nb_tiles; nb += NW) {
       fetch_a(nb, abuf[0]);
-      const uint32_t b = 16 * nb + i16;
 #pragma unroll
-      for (int s = 0; s < KSU; ++s)
-        if (4u * s + q4 >= U) abuf[0][s] = make_float2(0.f, 0.f);
+      for (int s = 0; s < KSU; ++s) {
+        if constexpr (QUAD)
+          abuf[0][s] = operand(abuf[0][s], s);
+        else if (4u * s + q4 >= U)
+          abuf[0][s] = make_float2(0.f, 0.f);
+      }
       // the -G^-1 reads are the same for every antenna tile: an offset the
       // compiler cannot see through (always 0) keeps it from holding all of
       // them in registers across tiles; the pointer itself stays sh.G's
@@ -547,27 +570,24 @@ __device__ __forceinline__ void zf_apply(const float2* A, uint32_t U, uint32_t B
                 if (!FULL && s % 4 == 0 && 4 * s >= (int)U) break;
                 const float2 m = rs[(16 * (m0 + mi) + i16) * LDG + 4 * s + q4];
                 const float gr = -m.x, gi = -m.y;
-                wr1 = mfma4(gr, abuf[0][s].x, wr1);
-                wr2 = mfma4(-gi, abuf[0][s].y, wr2);
-                wi1 = mfma4(gr, abuf[0][s].y, wi1);
-                wi2 = mfma4(gi, abuf[0][s].x, wi2);
+                wr1 = prod(abuf[0][s].x, gr, wr1);
+                wr2 = prod(abuf[0][s].y, -gi, wr2);
+                wi1 = prod(abuf[0][s].y, gr, wi1);
+                wi2 = prod(abuf[0][s].x, gi, wi2);
               }
             }
             rr[mi] = wr1 + wr2;
             ri[mi] = wi1 + wi2;
           }
-          if (b < B) {
+          const uint32_t b = 16 * nb + i16;
+          if constexpr (BROW) {
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi) store_tile(nb, m0 + mi, rr[mi], ri[mi]);
+          } else if (b < B) {
 #pragma unroll
             for (int mi = 0; mi < 2; ++mi)
 #pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const uint32_t u = 16 * (m0 + mi) + 4 * q4 + r;
-                if (u < U) {
-                  const float2 v = make_float2(rr[mi][r], ri[mi][r]);
-                  w[u + (uint64_t)ld_w * b] = v;
-                  if (w2) w2[u + (uint64_t)U * b] = v;
-                }
-              }
+              for (int r = 0; r < 4; ++r) put(16 * (m0 + mi) + 4 * q4 + r, b, rr[mi][r], ri[mi][r]);
           }
         }
       };

@@ -142,6 +142,29 @@ def test_zf_padded_user_tiles_are_bit_identical(U, B, G, tuning):
     assert np.abs(outs[0].view(np.complex64)).max() > 0
 
 
+@pytest.mark.parametrize("U,B,G", [(17, 33, 3), (30, 131, 2), (35, 70, 3), (63, 127, 2)])
+def test_zf_ragged_tiles_in_place(U, B, G):
+    """Users off the quads of four and antennas off the tiles of sixteen, in
+    which the weights' operand changes lanes: in place and out of place are the
+    same bits, and within the FP64 oracle's usual bound (condition numbers here
+    stay below 100: 100 * U * 2^-24 < 1e-3 of which 1e-4 is asked)."""
+    print(f"case: zf ragged U={U} B={B} G={G}", flush=True)
+    t = torch()
+    rng = np.random.Generator(np.random.Philox(U * 13 + B))
+    a = np.conj(synth.channel_iid(rng, G, B, U)).astype(np.complex64)
+    _, w64, _ = oracle.zf(a, U, B, G, "f64")
+    d, src = dev_c64(a.reshape(-1)), dev_c64(a.reshape(-1))
+    out = t.zeros_like(src)
+    m.zf(d, d, B, U, G)
+    m.zf(src, out, B, U, G)
+    _sync()
+    w = host_c64(out)
+    assert np.array_equal(host_c64(d).view(np.uint32), w.view(np.uint32))
+    ref = w64.reshape(G, B * U)
+    rel = np.linalg.norm(w.reshape(G, B * U) - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert rel.max() < 1e-4, rel.max()
+
+
 @pytest.mark.parametrize("U,B", [(8, 32), (100, 200)])
 def test_zf_in_place_and_failed_groups(U, B):
     print(f"case: zf in place with rank-deficient groups U={U} B={B}", flush=True)
