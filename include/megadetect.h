@@ -504,6 +504,34 @@ int mega_mlp_mse_grad(const float *Y, const float *T, float *dY, uint64_t n, uin
 int mega_mlp_adam(float *w, void *wb, const float *g, float *m, float *v, uint64_t n, float lr,
                   float beta1, float beta2, float eps, uint32_t step, mega_stream_t stream);
 int mega_mlp_to_bf16(const float *x, void *y, uint64_t n, mega_stream_t stream);
+/* mega_mlp_adam over several tensors (all of a network's) in one launch per
+ * eight. */
+typedef struct {
+  float *w;
+  void *wb;
+  const float *g;
+  float *m, *v;
+  uint64_t n;
+} mega_mlp_tensor;
+
+int mega_mlp_adam_group(const mega_mlp_tensor *t, uint32_t count, float lr, float beta1,
+                        float beta2, float eps, uint32_t step, mega_stream_t stream);
+/* The backward pass of `count` layers in one call, last layer first: per layer
+ * dZ = dY * act'(Z), gW = H^T dZ, gb = column sums of dZ, and (where dH is not
+ * NULL) dH = dZ W^T, the next one's dY. H, W, dZ are BF16 (M x n_in, n_in x
+ * n_out, M x n_out), all rows dense; dZf is the FP32 dZ's scratch (unused by
+ * identity layers). */
+typedef struct {
+  const void *H, *W;
+  const float *Z;
+  void *dZ;
+  float *dZf, *gW, *gb, *dH;
+  uint32_t n_in, n_out;
+  int32_t act;
+} mega_mlp_layer;
+
+int mega_mlp_backward(const mega_mlp_layer *layers, uint32_t count, uint32_t M, const float *dY,
+                      mega_stream_t stream);
 
 /* ---- LDPC consumer: decode the equalizer's code blocks ---------------------
  * Replaces LDPCDecoder(llr_type, LDPCConfig(mb, bg, Zc, max_iter)) and its

@@ -660,11 +660,44 @@ int mega_mlp_mse_grad(const float* Y, const float* T, float* dY, uint64_t n, uin
 
 int mega_mlp_adam(float* w, void* wb, const float* g, float* m, float* v, uint64_t n, float lr,
                   float beta1, float beta2, float eps, uint32_t step, mega_stream_t stream) {
-  if (n && (!w || !g || !m || !v || step == 0))
-    return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_adam: bad argument");
-  return hip_status(mega::detail::mlp_adam(w, static_cast<__bf16*>(wb), g, m, v, n, lr, beta1, beta2,
-                                           eps, step, static_cast<hipStream_t>(stream)),
+  const mega_mlp_tensor t{w, wb, g, m, v, n};
+  return mega_mlp_adam_group(&t, 1, lr, beta1, beta2, eps, step, stream);
+}
+
+int mega_mlp_adam_group(const mega_mlp_tensor* t, uint32_t count, float lr, float beta1,
+                        float beta2, float eps, uint32_t step, mega_stream_t stream) {
+  if (count && !t) return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_adam: NULL tensors");
+  for (uint32_t i = 0; i < count; ++i)
+    if (t[i].n && (!t[i].w || !t[i].g || !t[i].m || !t[i].v || step == 0))
+      return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_adam: bad argument");
+  return hip_status(mega::detail::mlp_adam(t, count, lr, beta1, beta2, eps, step,
+                                           static_cast<hipStream_t>(stream)),
                     "mega_mlp_adam");
+}
+
+int mega_mlp_backward(const mega_mlp_layer* layers, uint32_t count, uint32_t M, const float* dY,
+                      mega_stream_t stream) {
+  if (count && !layers) return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL layers");
+  for (uint32_t l = count; l-- > 0;) {
+    const mega_mlp_layer& y = layers[l];
+    const uint32_t ni = y.n_in, no = y.n_out;
+    if (!y.gW || !y.gb || (y.act != 0 && !y.dZf) || (l > 0 && !y.dH))
+      return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL buffer");
+    // an identity's FP32 dZ is dY itself
+    int rc = mega_mlp_act_backward(dY, y.Z, y.dZ, y.act ? y.dZf : nullptr, (uint64_t)M * no, y.act,
+                                   stream);
+    if (rc != MEGA_OK) return rc;
+    const mega_mlp_gemm_desc gw{y.H, 1, ni, y.dZ, no, 1, ni, no, M, nullptr, 0, y.gW, nullptr,
+                                no, 0.f};
+    if ((rc = mega_mlp_gemm(&gw, stream)) != MEGA_OK) return rc;
+    if ((rc = mega_mlp_col_sum(y.act ? y.dZf : dY, y.gb, M, no, stream)) != MEGA_OK) return rc;
+    if (!y.dH) continue;
+    const mega_mlp_gemm_desc dh{y.dZ, no, 1, y.W, 1, no, M, ni, no, nullptr, 0, y.dH, nullptr,
+                                ni, 0.f};
+    if ((rc = mega_mlp_gemm(&dh, stream)) != MEGA_OK) return rc;
+    dY = y.dH;
+  }
+  return MEGA_OK;
 }
 
 int mega_mlp_to_bf16(const float* x, void* y, uint64_t n, mega_stream_t stream) {

@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "megadetect.h"
+
 namespace mega {
 namespace detail {
 
@@ -29,8 +31,8 @@ hipError_t mlp_act_backward(const float* dY, const float* Z, __bf16* dZ, float* 
 hipError_t mlp_col_sum(const float* dZ, float* db, uint32_t M, uint32_t N, hipStream_t st);
 hipError_t mlp_mse_grad(const float* Y, const float* T, float* dY, uint64_t n, uint32_t M,
                         hipStream_t st);
-hipError_t mlp_adam(float* w, __bf16* wb, const float* g, float* m, float* v, uint64_t n,
-                    float lr, float b1, float b2, float eps, uint32_t step, hipStream_t st);
+hipError_t mlp_adam(const mega_mlp_tensor* t, uint32_t count, float lr, float b1, float b2,
+                    float eps, uint32_t step, hipStream_t st);
 hipError_t mlp_to_bf16(const float* x, __bf16* y, uint64_t n, hipStream_t st);
 
 }  // namespace detail

@@ -382,20 +382,32 @@ __global__ void mse_grad(const float* __restrict__ Y, const float* __restrict__ 
   dY[i] = (Y[i] - T[i]) * inv_m;
 }
 
-// Adam on FP32 master weights, BF16 copy for the GEMMs.
-__global__ void adam_step(float* __restrict__ w, __bf16* __restrict__ wb, const float* __restrict__ g,
-                          float* __restrict__ m, float* __restrict__ v, uint64_t n, float lr,
-                          float b1, float b2, float eps, float c1, float c2) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  w[i] = wi;
-  if (wb) wb[i] = (__bf16)wi;
+// Adam on FP32 master weights, BF16 copy for the GEMMs, over up to kAdamTensors
+// tensors: bound by memory (30 bytes a weight), but six launches a step of the
+// network, the biases' smaller than the gap before them, took 21.7 us where one
+// takes 11.9 (1.9 million weights).
+constexpr uint32_t kAdamTensors = 8, kAdamThreads = 256;
+struct AdamGroup {
+  mega_mlp_tensor t[kAdamTensors];
+  uint32_t end[kAdamTensors];  // workgroups up to and with tensor i
+};
+__global__ __launch_bounds__(kAdamThreads) void adam_step(const AdamGroup a, float lr, float b1,
+                                                          float b2, float eps, float c1,
+                                                          float c2) {
+  uint32_t k = 0;
+  while (blockIdx.x >= a.end[k]) ++k;  // uniform; the last one's is the grid's
+  const mega_mlp_tensor& t = a.t[k];
+  const uint64_t i =
+      (uint64_t)(blockIdx.x - (k ? a.end[k - 1] : 0u)) * kAdamThreads + threadIdx.x;
+  if (i >= t.n) return;
+  const float gi = t.g[i];
+  const float mi = b1 * t.m[i] + (1.f - b1) * gi;
+  const float vi = b2 * t.v[i] + (1.f - b2) * gi * gi;
+  t.m[i] = mi;
+  t.v[i] = vi;
+  const float wi = t.w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  t.w[i] = wi;
+  if (t.wb) static_cast<__bf16*>(t.wb)[i] = (__bf16)wi;
 }
 
 __global__ void to_bf16(const float* __restrict__ x, __bf16* __restrict__ y, uint64_t n) {
@@ -523,9 +535,8 @@ hipError_t mlp_mse_grad(const float* Y, const float* T, float* dY, uint64_t n, u
   return hipGetLastError();
 }
 
-hipError_t mlp_adam(float* w, __bf16* wb, const float* g, float* m, float* v, uint64_t n,
-                    float lr, float b1, float b2, float eps, uint32_t step, hipStream_t st) {
-  if (n == 0) return hipSuccess;
+hipError_t mlp_adam(const mega_mlp_tensor* t, uint32_t count, float lr, float b1, float b2,
+                    float eps, uint32_t step, hipStream_t st) {
   float c1 = 1.f, c2 = 1.f;
   for (uint32_t i = 0; i < step; ++i) {
     c1 *= b1;
@@ -533,8 +544,21 @@ hipError_t mlp_adam(float* w, __bf16* wb, const float* g, float* m, float* v, ui
   }
   c1 = 1.f - c1;
   c2 = 1.f - c2;
-  hipLaunchKernelGGL(adam_step, dim3(blocks_for(n, 256)), dim3(256), 0, st, w, wb, g, m, v, n,
-                     lr, b1, b2, eps, c1, c2);
+  for (uint32_t i = 0; i < count;) {
+    AdamGroup a;
+    uint32_t k = 0, blocks = 0;
+    for (; i < count && k < kAdamTensors; ++i) {
+      if (t[i].n == 0) continue;
+      const uint64_t nb = (t[i].n + kAdamThreads - 1) / kAdamThreads;
+      if (nb > 0x7fffffffu) return hipErrorInvalidConfiguration;
+      if (k && nb > 0x7fffffffu - blocks) break;  // the next launch's
+      a.t[k] = t[i];
+      a.end[k++] = blocks += (uint32_t)nb;
+    }
+    if (k == 0) break;
+    hipLaunchKernelGGL(adam_step, dim3(blocks), dim3(kAdamThreads), 0, st, a, lr, b1, b2, eps, c1,
+                       c2);
+  }
   return hipGetLastError();
 }
 

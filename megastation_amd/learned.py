@@ -36,6 +36,20 @@ class GemmDesc(ctypes.Structure):
                 ("Cb", ctypes.c_void_p), ("ldc", ctypes.c_uint32), ("beta", ctypes.c_float)]
 
 
+class Tensor(ctypes.Structure):
+    """Mirror of ``mega_mlp_tensor``."""
+    _fields_ = [("w", ctypes.c_void_p), ("wb", ctypes.c_void_p), ("g", ctypes.c_void_p),
+                ("m", ctypes.c_void_p), ("v", ctypes.c_void_p), ("n", ctypes.c_uint64)]
+
+
+class Layer(ctypes.Structure):
+    """Mirror of ``mega_mlp_layer``."""
+    _fields_ = [("H", ctypes.c_void_p), ("W", ctypes.c_void_p), ("Z", ctypes.c_void_p),
+                ("dZ", ctypes.c_void_p), ("dZf", ctypes.c_void_p), ("gW", ctypes.c_void_p),
+                ("gb", ctypes.c_void_p), ("dH", ctypes.c_void_p), ("n_in", ctypes.c_uint32),
+                ("n_out", ctypes.c_uint32), ("act", ctypes.c_int32)]
+
+
 _sig_done = False
 
 
@@ -57,6 +71,8 @@ def _L():
             "mega_mlp_mse_grad": [P, P, P, u64, u32, P],
             "mega_mlp_adam": [P, P, P, P, P, u64, f32, f32, f32, f32, u32, P],
             "mega_mlp_to_bf16": [P, P, u64, P],
+            "mega_mlp_adam_group": [P, u32, f32, f32, f32, f32, u32, P],
+            "mega_mlp_backward": [P, u32, u32, P, P],
         }
         for name, args in sig.items():
             f = getattr(L, name)
@@ -155,32 +171,37 @@ class WarmStartNet:
         import torch
         saved, zs, M = self._saved
         gw, gb = [None] * 3, [None] * 3
-        dy = dout
-        for l in (2, 1, 0):
+        # one native call for the 11 launches, the temporaries from one buffer:
+        # call by call a step of the 32-user network was bound by the host
+        layers = (Layer * 3)()
+        sizes = []  # per layer: BF16 dZ, FP32 dZ (identity: none), FP32 dH (first: none)
+        for l in range(3):
             n_in, n_out = self.dims[l], self.dims[l + 1]
-            dzb = torch.empty(M, n_out, dtype=torch.bfloat16, device="cuda")
-            dzf = torch.empty(M, n_out, device="cuda")
-            _check(_L().mega_mlp_act_backward(_ptr(dy), _ptr(zs[l]), _ptr(dzb), _ptr(dzf),
-                                              M * n_out, IDENTITY if l == 2 else GELU,
-                                              _stream(stream)))
+            sizes += [2 * M * n_out, 0 if l == 2 else 4 * M * n_out, 4 * M * n_in if l else 0]
+        at = [0]
+        for n in sizes:
+            at.append(at[-1] + (n + 255) // 256 * 256)
+        tmp = torch.empty(at[-1], dtype=torch.uint8, device="cuda")
+        base = tmp.data_ptr()
+        for l in range(3):
+            n_in, n_out = self.dims[l], self.dims[l + 1]
             gw[l] = torch.empty(n_in, n_out, device="cuda")
-            # dW = H^T dZ: A(i,k) = H[k][i]
-            gemm(saved[l], 1, n_in, dzb, n_out, 1, n_in, n_out, M, Cf=gw[l], stream=stream)
             gb[l] = torch.empty(n_out, device="cuda")
-            _check(_L().mega_mlp_col_sum(_ptr(dzf), _ptr(gb[l]), M, n_out, _stream(stream)))
-            if l > 0:
-                dy = torch.empty(M, n_in, device="cuda")
-                # dH = dZ W^T: B(k,j) = W[j][k]
-                gemm(dzb, n_out, 1, self.wb[l], 1, n_out, M, n_in, n_out, Cf=dy, stream=stream)
+            p = [base + at[3 * l + k] if sizes[3 * l + k] else None for k in range(3)]
+            layers[l] = Layer(saved[l].data_ptr(), self.wb[l].data_ptr(), zs[l].data_ptr(), p[0],
+                              p[1], gw[l].data_ptr(), gb[l].data_ptr(), p[2], n_in, n_out,
+                              IDENTITY if l == 2 else GELU)
+        _check(_L().mega_mlp_backward(layers, 3, M, _ptr(dout), _stream(stream)))
         self.grads = gw + gb
         return self.grads
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, stream=None):
         self.step += 1
+        t = (Tensor * len(self.params))()
         for k, (p, g, m, v) in enumerate(zip(self.params, self.grads, self.m, self.v)):
-            wb = self.wb[k] if k < 3 else None
-            _check(_L().mega_mlp_adam(_ptr(p), _ptr(wb), _ptr(g), _ptr(m), _ptr(v), p.numel(),
-                                      lr, b1, b2, eps, self.step, _stream(stream)))
+            t[k] = Tensor(p.data_ptr(), self.wb[k].data_ptr() if k < 3 else None, g.data_ptr(),
+                          m.data_ptr(), v.data_ptr(), p.numel())
+        _check(_L().mega_mlp_adam_group(t, len(t), lr, b1, b2, eps, self.step, _stream(stream)))
 
     def mse_grad(self, out, target, stream=None):
         import torch

@@ -95,6 +95,34 @@ def test_col_sum_is_four_running_sums(M, N):
     assert np.array_equal(db.cpu().numpy(), (p[0] + p[1]) + (p[2] + p[3]))
 
 
+@pytest.mark.parametrize("sizes", [(1,), (257, 0, 256, 1000), (3, 5, 70, 1, 0, 2, 300, 9, 11, 4)])
+def test_adam_group_equals_single_tensors(sizes):
+    """Several tensors a launch (empty ones, more than eight) against a call for
+    each: the same expressions on the same values, so the same bits."""
+    print(f"case: adam group {sizes}", flush=True)
+    t = torch()
+    g = t.Generator(device="cuda").manual_seed(sum(sizes))
+
+    def state():
+        g.manual_seed(sum(sizes))
+        r = [[t.rand(n, device="cuda", generator=g) for n in sizes] for _ in range(4)]
+        return (*r, [t.zeros(n, dtype=t.bfloat16, device="cuda") for n in sizes])
+    L = learned._L()
+    a, b = state(), state()
+    for step in (1, 2):
+        for w, gr, mm, v, wb in zip(*a):
+            m._check(L.mega_mlp_adam(m._ptr(w), m._ptr(wb), m._ptr(gr), m._ptr(mm), m._ptr(v),
+                                     w.numel(), 1e-3, 0.9, 0.999, 1e-8, step, m._stream(None)))
+        ts = (learned.Tensor * len(sizes))(*[
+            learned.Tensor(w.data_ptr(), wb.data_ptr(), gr.data_ptr(), mm.data_ptr(),
+                           v.data_ptr(), w.numel()) for w, gr, mm, v, wb in zip(*b)])
+        m._check(L.mega_mlp_adam_group(ts, len(sizes), 1e-3, 0.9, 0.999, 1e-8, step,
+                                       m._stream(None)))
+    for x, y in zip(a, b):
+        assert all(t.equal(p, q) for p, q in zip(x, y))
+    assert all(float(wb.abs().sum()) > 0 for wb in b[4] if wb.numel())
+
+
 def test_mlp_forward_backward_adam_match_oracle():
     print("case: mlp fwd/bwd/adam", flush=True)
     t = torch()
