@@ -150,52 +150,50 @@ __global__ __launch_bounds__(256) void gemm_bf16(const __bf16* __restrict__ A, i
       }
 }
 
-// ---- Direct GEMM: operands straight from global memory into registers -------
+// ---- Direct GEMM: operands from global memory into registers, wave by wave ----
 //
 // One workgroup owns one (16 FM) x (16 FN) tile of C. Where the staged kernel
 // splits K, a workgroup's waves take the splits' ranges and the partial tiles
 // are added in split order through LDS (no second kernel, no workspace): every
-// output is the same chain of MFMAs and sums, bit for bit. The shapes of the network (M 60-2112, N 512-2112, K 512-2112) are
-// bound by latency, not by the matrix cores or L2: a staged tile paid two
-// barriers and a transposing 2-byte LDS scatter per 32-wide step on one wave a
-// SIMD, here a wave keeps PD steps of both operands in flight and no wave waits
-// for another before the end.
+// output is the same chain of MFMAs and sums, bit for bit. The shapes of the
+// network (M 60-2112, N 512-2112, K 512-2112) give a SIMD one or two waves, so a
+// wave keeps PD steps of both operands in flight and no wave waits for another
+// before the end; the matrix cores are busy for less than a tenth of the time.
 //
-// An operand whose K index is the unit-stride one (KF) gives a lane its 8
-// consecutive K values as one 16-byte load per 16 rows. One whose row index is
-// (the weights' W[k][j], the transposed activations of dW) is loaded as F
-// consecutive rows of 8 K lines and the F fragments are put together with byte
-// permutes: fragment f then holds rows F*i + f instead of 16 f + i, which the
-// epilogue's row map undoes. Both operands use K = 8 (lane / 16) + v, the
-// order the MFMA sums over does not matter otherwise.
+// What bounds a step is how its operands reach the registers. In the order the
+// MFMA wants them (neighbour lanes in different rows) the load unit takes a
+// cycle a lane, 65 for a wave's 16-byte load, and 11.7 for one of 4 bytes: 223
+// cycles a step of 4 KB. So a lane loads 16 bytes with its neighbours' beside
+// them (17.5 cycles a load), and the wave exchanges them through its own few KB
+// of LDS, without a barrier. KF: K unit-stride, a row's 64 bytes to four lanes.
+// RF: rows unit-stride (the weights' W[k][j], the transposed activations of dW),
+// a K line's 16 F rows to 2 F lanes, read back by the transposing LDS loads.
+// RFN: rows unit-stride, but their count or pitch not in pieces of 8: F
+// consecutive rows of 8 K lines a lane, put together with byte permutes;
+// fragment f then holds rows F*i + f instead of 16 f + i, which the epilogue's
+// row map undoes. All use K = 8 (lane / 16) + v.
+// Operand order in registers only -> through LDS, us a call: 1092 x 512 x 2112
+// 21.4 -> 18.0, 2112 x 512 x 1092 T 22.3 -> 18.2, 16384 x 512 x 2112 122 -> 105.
 
-template <int F, bool KF>
+enum { KF, RF, RFN };  // an operand's unit-stride index and piece, as above
+
+template <int F, int S>
 struct GemmRaw {
-  static constexpr int W = KF ? 4 * F : 8 * (F / 2);  // words a lane holds
+  static constexpr int W = S == RFN ? 8 * (F / 2) : 4 * F;  // words a lane holds
   uint32_t w[W];
 };
 
-// Rows clamped to the last ones (their products are not stored); K lines past
-// K read as zero in the tail step.
-template <int F, bool KF, bool TAIL>
-__device__ __forceinline__ void gemm_load(GemmRaw<F, KF>& o, const __bf16* __restrict__ P,
+// One step's 32 K x 16 F rows. Rows clamped to the last ones (their products
+// are not stored); K past its end reads as zero in the tail step.
+template <int F, int S, bool TAIL>
+__device__ __forceinline__ void gemm_load(GemmRaw<F, S>& o, const __bf16* __restrict__ P,
                                           int64_t stride, uint32_t r0, uint32_t R, uint32_t k0,
-                                          uint32_t K, int i16, int q4) {
-  if constexpr (KF) {
-    const uint32_t k = k0 + 8 * q4;
-    const bool in = !TAIL || k < K;  // K % 8 == 0
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-      const uint32_t r = min(r0 + 16u * f + i16, R - 1);
-      uint4 v = *reinterpret_cast<const uint4*>(P + (int64_t)r * stride + (in ? k : 0u));
-      if (TAIL && !in) v = uint4{0, 0, 0, 0};
-      o.w[4 * f] = v.x, o.w[4 * f + 1] = v.y, o.w[4 * f + 2] = v.z, o.w[4 * f + 3] = v.w;
-    }
-  } else {
-    const uint32_t r = min(r0 + (uint32_t)F * i16, R - F);  // R % F == 0
+                                          uint32_t K, int lane) {
+  if constexpr (S == RFN) {
+    const uint32_t r = min(r0 + (uint32_t)F * (lane & 15), R - F);  // R % F == 0
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const uint32_t k = k0 + 8 * q4 + v;
+      const uint32_t k = k0 + 8 * (lane >> 4) + v;
       const bool in = !TAIL || k < K;
       const __bf16* p = P + (int64_t)(in ? k : 0u) * stride + r;
       if constexpr (F == 4) {
@@ -208,28 +206,74 @@ __device__ __forceinline__ void gemm_load(GemmRaw<F, KF>& o, const __bf16* __res
         o.w[v] = x;
       }
     }
+  } else {
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const int e = 64 * f + lane, line = e / (2 * F);  // RF: 2 F pieces a K line
+      const uint32_t k = k0 + (S == KF ? 8 * (lane % 4) : line);
+      const bool in = !TAIL || k < K;  // KF: K % 8 == 0
+      const uint32_t r = S == KF ? min(r0 + 16u * f + lane / 4, R - 1)
+                                 : min(r0 + 8u * (e % (2 * F)), R - 8);  // RF: R % 8 == 0
+      const uint32_t kc = in ? k : 0u;
+      uint4 v = *reinterpret_cast<const uint4*>(
+          S == KF ? P + (int64_t)r * stride + kc : P + (int64_t)kc * stride + r);
+      if (TAIL && !in) v = uint4{0, 0, 0, 0};
+      o.w[4 * f] = v.x, o.w[4 * f + 1] = v.y, o.w[4 * f + 2] = v.z, o.w[4 * f + 3] = v.w;
+    }
   }
 }
 
-template <int F, bool KF>
-__device__ __forceinline__ v8bf gemm_frag(const GemmRaw<F, KF>& o, int f) {
-  uint4 r;
-  if constexpr (KF) {
-    r = uint4{o.w[4 * f], o.w[4 * f + 1], o.w[4 * f + 2], o.w[4 * f + 3]};
+// The wave's copy of a loaded step in LDS (F KB): KF rows of 64 bytes, RF K
+// lines of 32 F bytes, their pieces exchanged so that neither these writes nor
+// the reads below meet in a bank.
+template <int F>
+__device__ __forceinline__ int rf_swap(int line) {
+  return F == 2 ? line >> 3 & 1 : (line >> 1 & 1) | (line >> 3 & 1) << 1;
+}
+template <int F, int S>
+__device__ __forceinline__ void gemm_stage(const GemmRaw<F, S>& o, char* L, int lane) {
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    const int e = 64 * f + lane, line = e / (2 * F), c = e % (2 * F);
+    const int at = S == KF ? 1024 * f + lane / 4 * 64 + (lane % 4 ^ lane >> 4) * 16
+                           : line * 32 * F + (c / 2 ^ rf_swap<F>(line)) * 32 + c % 2 * 16;
+    *reinterpret_cast<uint4*>(L + at) =
+        uint4{o.w[4 * f], o.w[4 * f + 1], o.w[4 * f + 2], o.w[4 * f + 3]};
+  }
+}
+
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s* LdsV4s;
+
+// Fragment f: this lane's row and its 8 K values.
+template <int F, int S>
+__device__ __forceinline__ v8bf gemm_frag(const GemmRaw<F, S>& o, char* L, int f, int lane) {
+  const int i16 = lane & 15, q4 = lane >> 4;
+  if constexpr (S == KF) {
+    return *reinterpret_cast<const v8bf*>(L + 1024 * f + i16 * 64 + (q4 ^ i16 >> 2) * 16);
+  } else if constexpr (S == RF) {
+    struct { v4s k[2]; } r;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // transposing reads of four K lines x 16 rows
+      const int line = 8 * q4 + 4 * h + i16 / 4;
+      r.k[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (LdsV4s)(L + line * 32 * F + (f ^ rf_swap<F>(line)) * 32 + i16 % 4 * 8));
+    }
+    return __builtin_bit_cast(v8bf, r);
   } else {
     // rows F i + f: half f % 2 of word f / 2 of each K line, two lines a word
     const uint32_t sel = f % 2 ? 0x07060302u : 0x05040100u;
     constexpr int H = F / 2;
     const int h = f / 2;
-    r = uint4{__builtin_amdgcn_perm(o.w[H * 1 + h], o.w[H * 0 + h], sel),
-              __builtin_amdgcn_perm(o.w[H * 3 + h], o.w[H * 2 + h], sel),
-              __builtin_amdgcn_perm(o.w[H * 5 + h], o.w[H * 4 + h], sel),
-              __builtin_amdgcn_perm(o.w[H * 7 + h], o.w[H * 6 + h], sel)};
+    return __builtin_bit_cast(
+        v8bf, uint4{__builtin_amdgcn_perm(o.w[H * 1 + h], o.w[H * 0 + h], sel),
+                    __builtin_amdgcn_perm(o.w[H * 3 + h], o.w[H * 2 + h], sel),
+                    __builtin_amdgcn_perm(o.w[H * 5 + h], o.w[H * 4 + h], sel),
+                    __builtin_amdgcn_perm(o.w[H * 7 + h], o.w[H * 6 + h], sel)});
   }
-  return __builtin_bit_cast(v8bf, r);
 }
 
-template <int FM, int FN, bool AKF, bool BKF>
+template <int FM, int FN, int SA, int SB>
 __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A, int64_t sa,
                                                    const __bf16* __restrict__ B, int64_t sb,
                                                    uint32_t M, uint32_t N, uint32_t K,
@@ -237,8 +281,8 @@ __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A,
                                                    float* __restrict__ Cf,
                                                    __bf16* __restrict__ Cb, uint32_t ldc,
                                                    float beta, int steps) {
-  constexpr int GM = 16 * FM, GN = 16 * FN, LD = GN + 4, PD = 3;  // 6: no faster
-  extern __shared__ float red[];  // [SK][GM][LD]
+  constexpr int GM = 16 * FM, GN = 16 * FN, LD = GN + 4, PD = FM == 4 ? 2 : 3;
+  extern __shared__ __align__(16) float red[];  // [SK][GM][LD]; before, a wave's staged steps
   const int lane = threadIdx.x & 63, i16 = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int SK = blockDim.x >> 6;
@@ -246,19 +290,32 @@ __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A,
   const int full = K / 32, first = wave * steps;
   const int n = min(full - first, steps);  // this wave's whole steps
   v4f acc[FM][FN] = {};
-  GemmRaw<FM, AKF> ra[PD];
-  GemmRaw<FN, BKF> rb[PD];
+  GemmRaw<FM, SA> ra[PD];
+  GemmRaw<FN, SB> rb[PD];
+  static_assert((FM + FN) * 1024 <= GM * LD * 4 && GM * LD % 4 == 0, "staged steps");
+  char* const La = reinterpret_cast<char*>(red + (size_t)wave * GM * LD);
+  char* const Lb = La + FM * 1024;
   auto load = [&](int d, int s) {
     const uint32_t k0 = 32u * (first + s);
-    gemm_load<FM, AKF, false>(ra[d], A, sa, m0, M, k0, K, i16, q4);
-    gemm_load<FN, BKF, false>(rb[d], B, sb, n0, N, k0, K, i16, q4);
+    gemm_load<FM, SA, false>(ra[d], A, sa, m0, M, k0, K, lane);
+    gemm_load<FN, SB, false>(rb[d], B, sb, n0, N, k0, K, lane);
+  };
+  // a wave's LDS accesses run in order: no more than their order in the code is
+  // needed between its own writes and reads
+  auto ordered = [] {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   };
   auto mul = [&](int d) {
+    if constexpr (SA != RFN) gemm_stage<FM, SA>(ra[d], La, lane);
+    if constexpr (SB != RFN) gemm_stage<FN, SB>(rb[d], Lb, lane);
+    ordered();
     v8bf a[FM], b[FN];
 #pragma unroll
-    for (int f = 0; f < FM; ++f) a[f] = gemm_frag<FM, AKF>(ra[d], f);
+    for (int f = 0; f < FM; ++f) a[f] = gemm_frag<FM, SA>(ra[d], La, f, lane);
 #pragma unroll
-    for (int f = 0; f < FN; ++f) b[f] = gemm_frag<FN, BKF>(rb[d], f);
+    for (int f = 0; f < FN; ++f) b[f] = gemm_frag<FN, SB>(rb[d], Lb, f, lane);
+    ordered();
 #pragma unroll
     for (int x = 0; x < FM; ++x)
 #pragma unroll
@@ -283,8 +340,8 @@ __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A,
       if (s + d < n) mul(d);
   }
   if (K % 32 && wave == SK - 1) {  // the tail step ends the last range
-    gemm_load<FM, AKF, true>(ra[0], A, sa, m0, M, 32u * full, K, i16, q4);
-    gemm_load<FN, BKF, true>(rb[0], B, sb, n0, N, 32u * full, K, i16, q4);
+    gemm_load<FM, SA, true>(ra[0], A, sa, m0, M, 32u * full, K, lane);
+    gemm_load<FN, SB, true>(rb[0], B, sb, n0, N, 32u * full, K, lane);
     mul(0);
   }
   // D lane l, reg r = fragment row 4 (l / 16) + r, column l % 16
@@ -292,10 +349,10 @@ __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A,
   for (int x = 0; x < FM; ++x)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = AKF ? 16 * x + 4 * q4 + r : FM * (4 * q4 + r) + x;
+      const int i = SA != RFN ? 16 * x + 4 * q4 + r : FM * (4 * q4 + r) + x;
       float* o = red + ((size_t)wave * GM + i) * LD;
 #pragma unroll
-      for (int y = 0; y < FN; ++y) o[BKF ? 16 * y + i16 : FN * i16 + y] = acc[x][y][r];
+      for (int y = 0; y < FN; ++y) o[SB != RFN ? 16 * y + i16 : FN * i16 + y] = acc[x][y][r];
     }
   __syncthreads();
   for (int e = threadIdx.x; e < GM * GN; e += blockDim.x) {
@@ -419,39 +476,46 @@ uint32_t blocks_for(uint64_t n, uint32_t t) { return (uint32_t)((n + t - 1) / t)
 
 }  // namespace
 
-// An operand the direct kernel can load in whole vectors: K unit-stride with
-// 16-byte rows, or rows unit-stride in pieces of f.
-bool direct_kf(const __bf16* p, int64_t sr, int64_t sk, uint32_t K) {
-  return sk == 1 && sr % 8 == 0 && K % 8 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-}
-bool direct_rf(const __bf16* p, int64_t sr, int64_t sk, uint32_t R, uint32_t f) {
-  return sr == 1 && sk % f == 0 && R % f == 0 && reinterpret_cast<uintptr_t>(p) % (2 * f) == 0;
+// How the direct kernel can load an operand in whole vectors (R rows, tiles of
+// 16 f), or -1.
+int direct_src(const __bf16* p, int64_t sr, int64_t sk, uint32_t R, uint32_t K, uint32_t f) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+  auto rows = [&](uint32_t v) { return sr == 1 && sk % v == 0 && R % v == 0 && at % (2 * v) == 0; };
+  if (sk == 1 && sr % 8 == 0 && K % 8 == 0 && at % 16 == 0) return KF;
+  return rows(8) ? RF : rows(f) ? RFN : -1;
 }
 
-template <int FM, int FN, bool AKF, bool BKF>
+template <int FM, int FN, int SA, int SB>
 hipError_t direct_run(const MlpGemm& g, uint32_t sk, uint32_t kchunk, hipStream_t st) {
   constexpr uint32_t GM = 16 * FM, GN = 16 * FN;
   const uint32_t lds = sk * GM * (GN + 4) * sizeof(float);
+  const auto fn = &gemm_direct<FM, FN, SA, SB>;
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&gemm_direct<FM, FN, AKF, BKF>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
   const dim3 grid((g.N + GN - 1) / GN, (g.M + GM - 1) / GM);
-  hipLaunchKernelGGL((gemm_direct<FM, FN, AKF, BKF>), grid, dim3(64 * sk), lds, st, g.A,
-                     AKF ? g.sai : g.sak, g.B, BKF ? g.sbj : g.sbk, g.M, g.N, g.K, g.bias, g.act,
-                     g.Cf, g.Cb, g.ldc, g.beta, (int)(kchunk / TK));
+  hipLaunchKernelGGL(fn, grid, dim3(64 * sk), lds, st, g.A, SA == KF ? g.sai : g.sak, g.B,
+                     SB == KF ? g.sbj : g.sbk, g.M, g.N, g.K, g.bias, g.act, g.Cf, g.Cb, g.ldc,
+                     g.beta, (int)(kchunk / TK));
   return hipGetLastError();
 }
 
-template <int FM, int FN>
-hipError_t direct_pick(const MlpGemm& g, bool akf, bool bkf, uint32_t sk, uint32_t kc,
+template <int FM, int FN, int SA>
+hipError_t direct_pick_b(const MlpGemm& g, int sb, uint32_t sk, uint32_t kc, hipStream_t st) {
+  return sb == KF   ? direct_run<FM, FN, SA, KF>(g, sk, kc, st)
+         : sb == RF ? direct_run<FM, FN, SA, RF>(g, sk, kc, st)
+                    : direct_run<FM, FN, SA, RFN>(g, sk, kc, st);
+}
+
+template <int F>
+hipError_t direct_pick(const MlpGemm& g, int sa, int sb, uint32_t sk, uint32_t kc,
                        hipStream_t st) {
-  return akf ? (bkf ? direct_run<FM, FN, true, true>(g, sk, kc, st)
-                    : direct_run<FM, FN, true, false>(g, sk, kc, st))
-             : (bkf ? direct_run<FM, FN, false, true>(g, sk, kc, st)
-                    : direct_run<FM, FN, false, false>(g, sk, kc, st));
+  return sa == KF   ? direct_pick_b<F, F, KF>(g, sb, sk, kc, st)
+         : sa == RF ? direct_pick_b<F, F, RF>(g, sb, sk, kc, st)
+                    : direct_pick_b<F, F, RFN>(g, sb, sk, kc, st);
 }
 
 // K splits: enough workgroups to cover the CUs (>= 256) while every split
@@ -462,10 +526,11 @@ hipError_t direct_pick(const MlpGemm& g, bool akf, bool bkf, uint32_t sk, uint32
 // being captured into a graph.
 hipError_t mlp_gemm(const MlpGemm& g, hipStream_t st) {
   if (g.M == 0 || g.N == 0) return hipSuccess;
-  const bool akf = direct_kf(g.A, g.sai, g.sak, g.K), bkf = direct_kf(g.B, g.sbj, g.sbk, g.K);
-  auto fits = [&](uint32_t fm, uint32_t fn) {
-    return (akf || direct_rf(g.A, g.sai, g.sak, g.M, fm)) &&
-           (bkf || direct_rf(g.B, g.sbj, g.sbk, g.N, fn));
+  int sa = -1, sb = -1;
+  auto fits = [&](uint32_t f) {
+    sa = direct_src(g.A, g.sai, g.sak, g.M, g.K, f);
+    sb = direct_src(g.B, g.sbj, g.sbk, g.N, g.K, f);
+    return sa >= 0 && sb >= 0;
   };
   const uint32_t tiles = ((g.N + TN - 1) / TN) * ((g.M + TM - 1) / TM);
   const uint32_t ksteps = (g.K + TK - 1) / TK;
@@ -476,22 +541,21 @@ hipError_t mlp_gemm(const MlpGemm& g, hipStream_t st) {
   // Direct kernel wherever both operands load in whole vectors and the splits
   // fit a workgroup. 32 x 32 tiles spread the network's own shapes over the
   // CUs; they read each operand once per 32 rows, so grids of 64 x 64 tiles
-  // that fill the chip several times over take those instead (L2-bound).
+  // that fill the chip several times over take those instead.
   // Measured, us a call, staged kernel (+ reduce) / 32 x 32 / 64 x 64 (M x N x K,
   // T: both operands' rows unit-stride; a call costs 8 us to issue):
-  //   273 x 512 x 2112      18.2 /  9.0 / 20.1
-  //   1092 x 512 x 2112     40.8 / 22.8 / 34.0
-  //   2112 x 512 x 1092 T    107 / 24.9 / 43.7
-  //   4368 x 512 x 512      40.0 / 26.8 / 36.2   (552 tiles of 64 x 64)
-  //   16384 x 512 x 512     81.6 / 73.4 / 59.0   (2048)
-  //   16384 x 512 x 2112     200 /  226 /  121   (2048)
-  //   2112 x 512 x 16384 T  1486 /  238 /  320   (264)
+  //   273 x 512 x 2112      18.2 /  8.9 / 13.9
+  //   1092 x 512 x 2112     40.8 / 18.0 / 21.4
+  //   2112 x 512 x 1092 T    107 / 18.2 / 26.3
+  //   4368 x 512 x 512      40.0 / 16.2 / 23.3   (552 tiles of 64 x 64)
+  //   8192 x 512 x 512         - / 23.5 / 27.0   (1024)
+  //   16384 x 512 x 512     81.6 / 42.6 / 38.0   (2048)
+  //   16384 x 512 x 2112     200 /  182 /  107   (2048)
+  //   2112 x 512 x 16384 T  1486 /  236 /  185   (264)
   if (splits <= 8) {
     const uint64_t tiles64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (tiles64 >= 1024 && fits(4, 4))
-      return direct_pick<4, 4>(g, akf, bkf, splits, kchunk, st);
-    if ((g.M + 31) / 32 <= 65535 && fits(2, 2))
-      return direct_pick<2, 2>(g, akf, bkf, splits, kchunk, st);
+    if (tiles64 >= 1024 && fits(4)) return direct_pick<4>(g, sa, sb, splits, kchunk, st);
+    if ((g.M + 31) / 32 <= 65535 && fits(2)) return direct_pick<2>(g, sa, sb, splits, kchunk, st);
   }
   float* part = nullptr;
   if (splits > 1) {

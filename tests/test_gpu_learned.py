@@ -51,7 +51,8 @@ def test_gemm_strided_transposes(M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(273, 512, 2112), (60, 512, 76), (36, 68, 24), (34, 62, 1092),
-                                   (2084, 2048, 72)])
+                                   (2084, 2048, 72), (72, 40, 100), (40, 264, 1000),
+                                   (2056, 2048, 104)])
 def test_gemm_direct_equals_staged(M, N, K):
     """The register kernel (operands whose rows load in whole vectors) against
     the staged one, which the same operands two bytes off the vector grid
