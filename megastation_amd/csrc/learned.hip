@@ -159,14 +159,44 @@ __global__ __launch_bounds__(256) void refine_kernel(
   __shared__ float red[4];
   const uint32_t g = blockIdx.x;
   const uint64_t o = (uint64_t)g * U * U;
-  for (int e = threadIdx.x; e < UP * UP; e += L::NTH) {
-    const int i = e / UP, c = e % UP;
-    const bool in = i < (int)U && c < (int)U;
-    const float2 a = in ? G[o + i * U + c] : make_float2(0.f, 0.f);
-    const float2 b = in ? Gp[o + i * U + c] : make_float2(0.f, 0.f);
-    sG[i * LD + c] = a;
-    sT[i * LD + c] = make_float2(a.x - b.x, a.y - b.y);  // D
-    sX[i * LD + c] = in ? Xp[o + i * U + c] : make_float2(0.f, 0.f);
+  // Bound by the latency of a group (a CU's only one): every load goes out
+  // before the first is used, from clamped addresses (a branch around them costs
+  // a round trip each), and the correction's arrive during the first products:
+  // 16.9 -> 13.8 us for 273 groups of 32 users, 4.2 of them FP32 products.
+  constexpr int E = UP * UP / L::NTH, EC = E < 4 ? E : 4;
+  const float* cg = corr ? corr + (uint64_t)g * corr_ld : nullptr;
+  const float sc = corr ? scale[g] : 1.f;
+  float2 cv[E];
+  const float2 zero = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int q0 = 0; q0 < E; q0 += EC) {
+    float2 a[EC], b[EC], x[EC];
+#pragma unroll
+    for (int q = 0; q < EC; ++q) {
+      const uint32_t e = threadIdx.x + (q0 + q) * L::NTH;
+      const uint64_t at = o + min(e / UP, U - 1) * U + min(e % UP, U - 1);
+      a[q] = G[at];
+      b[q] = Gp[at];
+      x[q] = Xp[at];
+    }
+    if (q0 + EC == E && cg) {
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const uint32_t e = threadIdx.x + q * L::NTH;
+        const uint32_t i = min(e / UP, U - 1), c = min(e % UP, U - 1);
+        const uint32_t m = min(i, c), n = max(i, c);
+        const uint32_t t = m * U - m * (m - 1) / 2 + (n - m);  // upper-triangle index
+        cv[q] = make_float2(cg[2 * t], cg[2 * t + 1]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < EC; ++q) {
+      const int e = threadIdx.x + (q0 + q) * L::NTH, i = e / UP, c = e % UP;
+      const bool in = i < (int)U && c < (int)U;
+      sG[i * LD + c] = in ? a[q] : zero;
+      sT[i * LD + c] = in ? make_float2(a[q].x - b[q].x, a[q].y - b[q].y) : zero;  // D
+      sX[i * LD + c] = in ? x[q] : zero;
+    }
   }
   __syncthreads();
   auto store = [](float2* M) {
@@ -177,16 +207,14 @@ __global__ __launch_bounds__(256) void refine_kernel(
   cmm<UP>(sV, sX, store(sT));  // Xp D Xp
   __syncthreads();
   // X0 = Xp - Xp D Xp + C / s (C Hermitian from its upper triangle)
-  const float inv = corr ? 1.f / scale[g] : 0.f;
-  const float* cg = corr ? corr + (uint64_t)g * corr_ld : nullptr;
-  for (int e = threadIdx.x; e < UP * UP; e += L::NTH) {
-    const int i = e / UP, c = e % UP;
+  const float inv = corr ? 1.f / sc : 0.f;
+#pragma unroll
+  for (int q = 0; q < E; ++q) {
+    const int e = threadIdx.x + q * L::NTH, i = e / UP, c = e % UP;
     float cr = 0.f, ci = 0.f;
     if (cg && i < (int)U && c < (int)U) {
-      const uint32_t a = min(i, c), b = max(i, c);
-      const uint32_t t = a * U - a * (a - 1) / 2 + (b - a);  // upper-triangle index
-      cr = cg[2 * t] * inv;
-      ci = i > c ? -cg[2 * t + 1] * inv : i == c ? 0.f : cg[2 * t + 1] * inv;
+      cr = cv[q].x * inv;
+      ci = i > c ? -cv[q].y * inv : i == c ? 0.f : cv[q].y * inv;
     }
     const float2 x = sX[i * LD + c], d = sT[i * LD + c];
     sX[i * LD + c] = make_float2(x.x - d.x + cr, x.y - d.y + ci);
