@@ -534,10 +534,10 @@ hipError_t mlp_gemm(const MlpGemm& g, hipStream_t st) {
   };
   const uint32_t tiles = ((g.N + TN - 1) / TN) * ((g.M + TM - 1) / TM);
   const uint32_t ksteps = (g.K + TK - 1) / TK;
-  uint32_t splits = 1;
+  uint32_t splits = 1;  // an empty sum (K = 0) is one split of no steps: the epilogue alone
   while (tiles * splits < 256 && ksteps / (splits + 1) >= 8) ++splits;
-  const uint32_t kchunk = ((ksteps + splits - 1) / splits) * TK;
-  splits = (g.K + kchunk - 1) / kchunk;
+  const uint32_t kchunk = ksteps ? ((ksteps + splits - 1) / splits) * TK : TK;
+  splits = ksteps ? (g.K + kchunk - 1) / kchunk : 1;
   // Direct kernel wherever both operands load in whole vectors and the splits
   // fit a workgroup. 32 x 32 tiles spread the network's own shapes over the
   // CUs; they read each operand once per 32 rows, so grids of 64 x 64 tiles

@@ -82,6 +82,20 @@ def test_gemm_direct_equals_staged(M, N, K):
             assert t.equal(got[0][0], got[1][0]) and t.equal(got[0][1], got[1][1]), (a_t, b_t)
 
 
+@pytest.mark.parametrize("M,N", [(64, 64), (33, 70)])  # the register and the staged kernel
+def test_gemm_of_an_empty_sum_is_its_epilogue(M, N):
+    """K = 0: no operand is read, C is the bias (and beta times what it held)."""
+    print(f"case: gemm K=0 M={M} N={N}", flush=True)
+    t = torch()
+    a = t.full((8,), float("nan"), dtype=t.bfloat16, device="cuda")
+    bias = t.arange(N, dtype=t.float32, device="cuda")
+    C = t.full((M, N), 2.0, device="cuda")
+    Cb = t.full((M, N), 2.0, dtype=t.bfloat16, device="cuda")
+    learned.gemm(a, 1, M, a, N, 1, M, N, 0, bias=bias, Cf=C, Cb=Cb, beta=0.5)
+    assert t.equal(C, (bias + 1.0).expand(M, N))
+    assert t.equal(Cb, bias.to(t.bfloat16).expand(M, N))
+
+
 @pytest.mark.parametrize("M,N", [(1, 5), (3, 16), (1024, 17), (1025, 40), (2111, 33)])
 def test_col_sum_is_four_running_sums(M, N):
     print(f"case: col_sum M={M} N={N}", flush=True)
