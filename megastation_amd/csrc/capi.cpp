@@ -626,11 +626,13 @@ int mega_learned_finish(uint32_t num_bs, uint32_t num_ue, uint32_t batch, const 
                     "mega_learned_finish");
 }
 
+static constexpr uint32_t kMaxGemmRows = 65535u * 64u;  // the grid's rows of 64-row tiles
+
 int mega_mlp_gemm(const mega_mlp_gemm_desc* d, mega_stream_t stream) {
   if (!d || !d->A || !d->B || (!d->Cf && !d->Cb))
     return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_gemm: NULL buffer");
   if (d->act != 0 && d->act != 1) return fail(MEGA_ERR_UNSUPPORTED, "mega_mlp_gemm: activation");
-  if (d->M > 65535u * 64u) return fail(MEGA_ERR_UNSUPPORTED, "mega_mlp_gemm: M too large");
+  if (d->M > kMaxGemmRows) return fail(MEGA_ERR_UNSUPPORTED, "mega_mlp_gemm: M too large");
   mega::detail::MlpGemm g{static_cast<const __bf16*>(d->A), d->sai, d->sak,
                           static_cast<const __bf16*>(d->B), d->sbk, d->sbj, d->M, d->N, d->K,
                           d->bias, d->act, d->Cf, static_cast<__bf16*>(d->Cb), d->ldc, d->beta};
@@ -677,12 +679,23 @@ int mega_mlp_adam_group(const mega_mlp_tensor* t, uint32_t count, float lr, floa
 
 int mega_mlp_backward(const mega_mlp_layer* layers, uint32_t count, uint32_t M, const float* dY,
                       mega_stream_t stream) {
-  if (count && !layers) return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL layers");
+  if (count && (!layers || !dY)) return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL buffer");
+  // every layer before the first launch: a refused call writes nothing
+  for (uint32_t l = 0; l < count; ++l) {
+    const mega_mlp_layer& y = layers[l];
+    if (!y.H || !y.Z || !y.dZ || !y.gW || !y.gb || (y.act != 0 && !y.dZf) || (l > 0 && !y.dH) ||
+        (y.dH && !y.W))
+      return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL buffer");
+    if (y.act != 0 && y.act != 1) return fail(MEGA_ERR_UNSUPPORTED, "mega_mlp_backward: activation");
+    if (y.n_in > kMaxGemmRows || (y.dH && M > kMaxGemmRows))
+      return fail(MEGA_ERR_UNSUPPORTED, "mega_mlp_backward: M too large");
+    // layer l's input is layer l - 1's output
+    if (l > 0 && y.n_in != layers[l - 1].n_out)
+      return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: layer widths do not chain");
+  }
   for (uint32_t l = count; l-- > 0;) {
     const mega_mlp_layer& y = layers[l];
     const uint32_t ni = y.n_in, no = y.n_out;
-    if (!y.gW || !y.gb || (y.act != 0 && !y.dZf) || (l > 0 && !y.dH))
-      return fail(MEGA_ERR_INVALID_ARG, "mega_mlp_backward: NULL buffer");
     // an identity's FP32 dZ is dY itself
     int rc = mega_mlp_act_backward(dY, y.Z, y.dZ, y.act ? y.dZf : nullptr, (uint64_t)M * no, y.act,
                                    stream);

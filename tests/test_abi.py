@@ -181,3 +181,32 @@ def test_bad_ldpc_arguments_rejected_before_launch():
         assert call(**kw) == code, kw
         assert msg in m.last_error(), (kw, m.last_error())
     assert call(num_cb=0) == m.MEGA_OK          # nothing to decode
+
+
+def _mlp_layers():
+    """Two chained layers of stand-in pointers (nothing is launched)."""
+    from megastation_amd import learned
+    p = 4096
+    return (learned.Layer * 2)(
+        learned.Layer(p, p, p, p, p, p, p, None, 8, 16, learned.GELU),
+        learned.Layer(p, p, p, p, None, p, p, p, 16, 4, learned.IDENTITY))
+
+
+@pytest.mark.parametrize("layer,field,value,code", [
+    *((0, f, None, m.MEGA_ERR_INVALID_ARG) for f in ("H", "Z", "dZ", "dZf", "gW", "gb")),
+    *((1, f, None, m.MEGA_ERR_INVALID_ARG) for f in ("H", "W", "Z", "dZ", "gW", "gb", "dH")),
+    (0, "act", 2, m.MEGA_ERR_UNSUPPORTED), (0, "n_in", 65535 * 64 + 1, m.MEGA_ERR_UNSUPPORTED),
+    (1, "n_in", 15, m.MEGA_ERR_INVALID_ARG)])
+def test_bad_mlp_layer_is_rejected_before_the_first_launch(layer, field, value, code):
+    """The layers run last first, so a bad first layer must not be found after
+    the others' gradients are written. (Without a GPU a launch is a HIP error.)"""
+    from megastation_amd import learned
+    layers = _mlp_layers()
+    setattr(layers[layer], field, value)
+    assert learned._L().mega_mlp_backward(layers, 2, 3, ctypes.c_void_p(4096), None) == code
+    assert "mega_mlp_backward" in m.last_error()
+
+
+def test_mlp_backward_without_an_output_gradient_is_rejected():
+    from megastation_amd import learned
+    assert learned._L().mega_mlp_backward(_mlp_layers(), 2, 3, None, None) == m.MEGA_ERR_INVALID_ARG
