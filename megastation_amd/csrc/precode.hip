@@ -67,14 +67,13 @@ __global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint
   float p1[J][NACC], p2[J][NACC];
   // antennas past B and users past U clamped (dropped rows, zero symbols)
   auto load_p = [&](uint32_t gg) {
-    const char* P = reinterpret_cast<const char*>(a.prec + (uint64_t)gg * U * B);
+    const float2* P = a.prec + (uint64_t)gg * U * B;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const uint32_t row = min(4u * j + q, U - 1) * B;
+      const float2* row = P + (uint64_t)min(4u * j + q, U - 1) * B;
 #pragma unroll
       for (int m = 0; m < NACC; ++m) {
-        const uint32_t e = row + min(b0 + 8u * m + (i16 >> 1), B - 1);
-        const float2 v = *reinterpret_cast<const float2*>(P + e * 8u);
+        const float2 v = row[min(b0 + 8u * m + (i16 >> 1), B - 1)];
         p1[j][m] = h ? v.y : v.x;
         p2[j][m] = h ? v.x : -v.y;
       }
@@ -83,7 +82,7 @@ __global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint
   // user symbols of column 16 t + i16 (past the group: its last column, whose
   // results are dropped), users 4 j + q
   auto load_x = [&](uint32_t gg, uint32_t tt, float2 (&x)[J]) {
-    const uint32_t n = min(16 * tt + i16, ncol - 1), s = n / sg;
+    const uint32_t n = 16 * tt + min((uint32_t)i16, ncol - 1 - 16 * tt), s = n / sg;
     const float2* xcol = a.ue + (uint64_t)s * a.ue_sym + (uint64_t)gg * sg + (n - s * sg);
 #pragma unroll
     for (int j = 0; j < J; ++j) x[j] = xcol[(uint64_t)min(4u * j + q, U - 1) * N];
@@ -144,7 +143,9 @@ __global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint
       col -= col >= row ? row : 0;
     else
       col %= row;
-    O = n < ncol ? a.out + (uint64_t)s * a.out_sym + col + (uint64_t)(b0 + 2 * q) * row : nullptr;
+    O = (uint32_t)i16 < ncol - 16 * t
+            ? a.out + (uint64_t)s * a.out_sym + col + (uint64_t)(b0 + 2 * q) * row
+            : nullptr;
     if (++t == ntile) {
       t = 0;
       ++g;
@@ -188,7 +189,7 @@ hipError_t launch_precode(const PrecodeArgs& a, hipStream_t st, const char** why
     return hipErrorInvalidValue;
   }
   const uint64_t G = a.N / a.sg;  // full groups only, as the reference
-  if ((uint64_t)a.sg * a.S > 0xfffffff0ull) {
+  if ((uint64_t)a.sg * a.S > 0xffffffffull) {
     *why = "grid too large";
     return hipErrorInvalidValue;
   }

@@ -106,6 +106,21 @@ def test_bad_precode_arguments():
     assert ctypes.sizeof(m.PrecodeDesc) == 80
 
 
+@pytest.mark.parametrize("cols,refused", [(2**32 - 1, False), (2**32 - 16, False), (2**32, True)])
+def test_precode_columns_of_a_group_are_bounded_by_32_bits(cols, refused):
+    """Stand-in pointers, so only where nothing can be launched: an accepted
+    call ends at the missing device."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("would launch on stand-in pointers")
+    sg = 1 << 16 if cols % (1 << 16) == 0 else 3 if cols % 3 == 0 else 16
+    p = ctypes.c_void_p(4096).value
+    d = m.PrecodeDesc(1, 1, sg, sg, cols // sg, sg, 0, p, p, sg, p, sg)
+    assert m.lib().mega_precode_syms(ctypes.byref(d), None) == m.MEGA_ERR_HIP
+    assert ("grid too large" in m.last_error()) == refused
+
+
+
 @pytest.mark.parametrize("n", [16, 32, 1200, 3276])
 def test_pilot_sign_matches_oracle_bit_for_bit(n):
     """mega_pilot_sign (host) against the oracle's restatement of

@@ -99,6 +99,24 @@ def test_precode_ranges_match_fp64(B, U, N, sg, row, start, S):
     assert (np.abs(got - exp) <= 4 * U * 2.0 ** -23 * mag + 1e-30).all()
 
 
+def test_precode_group_beyond_32_bit_byte_offsets():
+    """One group's precoder of 4 GiB and a little: antennas past 2^29 read their
+    own entries (times 2: exact)."""
+    B = 2**29 + 40
+    print(f"case: precode B={B} U=1", flush=True)
+    t = torch()
+    P = t.zeros(B, 2, device="cuda:0")
+    P[:, 0] = t.arange(B, device="cuda:0", dtype=t.float32)
+    P[:, 1] = 1.0
+    ue = t.full((1,), 2.0 + 0j, dtype=t.complex64, device="cuda:0")
+    out = t.full((B, 2), -1.0, device="cuda:0")
+    m.precode(P, ue, out, num_bs=B, num_ue=1, num_sc=1, sc_group=1, bs_stride=1, bs_start=0,
+              num_syms=1)
+    P *= 2
+    for lo in range(0, B, 2**26):
+        assert t.equal(out[lo:lo + 2**26], P[lo:lo + 2**26]), lo
+
+
 @pytest.mark.parametrize("U,B,G", [(1, 1, 3), (32, 256, 5), (64, 256, 2), (128, 300, 2), (100, 1, 4),
                                    (17000, 2, 1)])
 def test_precoder_normalisation_shapes(U, B, G):
