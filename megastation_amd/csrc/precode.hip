@@ -65,7 +65,8 @@ __global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint
   uint32_t g = (uint32_t)(w / ntile), t = (uint32_t)(w % ntile);
   constexpr int PD = 2;
   float p1[J][NACC], p2[J][NACC];
-  // antennas past B and users past U clamped (dropped rows, zero symbols)
+  // antennas past B clamped (dropped rows), users past U zeros, as their
+  // symbols are: an infinity on either side of a zero would be a NaN
   auto load_p = [&](uint32_t gg) {
     const float2* P = a.prec + (uint64_t)gg * U * B;
 #pragma unroll
@@ -73,7 +74,8 @@ __global__ __launch_bounds__(256, 2) void precode_mfma(const PrecodeArgs a, uint
       const float2* row = P + (uint64_t)min(4u * j + q, U - 1) * B;
 #pragma unroll
       for (int m = 0; m < NACC; ++m) {
-        const float2 v = row[min(b0 + 8u * m + (i16 >> 1), B - 1)];
+        float2 v = row[min(b0 + 8u * m + (i16 >> 1), B - 1)];
+        if (4u * j + q >= U) v = make_float2(0.f, 0.f);
         p1[j][m] = h ? v.y : v.x;
         p2[j][m] = h ? v.x : -v.y;
       }

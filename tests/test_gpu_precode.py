@@ -99,6 +99,33 @@ def test_precode_ranges_match_fp64(B, U, N, sg, row, start, S):
     assert (np.abs(got - exp) <= 4 * U * 2.0 ** -23 * mag + 1e-30).all()
 
 
+@pytest.mark.parametrize("U,B", [(2, 40), (6, 200), (17, 64), (18, 130), (34, 70)])
+def test_precode_infinities_of_the_last_user(U, B):
+    """Users are padded to whole steps: an infinite entry or symbol of the last
+    one gives the products' infinities, not the NaN of a padded zero times it."""
+    print(f"case: precode infinities U={U} B={B}", flush=True)
+    rng = np.random.default_rng(U)
+    N, sg = 48, 12
+    t = torch()
+    draw = lambda *s: (rng.standard_normal(s) + 1j * rng.standard_normal(s)).astype(np.complex64)
+    P, ue = draw(N // sg, U, B), draw(1, U, N)
+    P[1, U - 1, ::3] = np.inf + 1j
+    ue[0, U - 1, 30::5] = complex(2, -np.inf)
+    out = t.zeros(B, N, dtype=t.complex64, device="cuda:0")
+    m.precode(dev_c64(P.reshape(-1)), dev_c64(ue.reshape(-1)), out, num_bs=B, num_ue=U, num_sc=N,
+              sc_group=sg, bs_stride=N, bs_start=N // 2, num_syms=1)
+    got = host_c64(out).reshape(B, N)
+    Pk = np.repeat(P, sg, axis=0).astype(np.complex128)       # [N][U][B]
+    x = ue[0].T[:, :, None].astype(np.complex128)             # [N][U][1]
+    re = (Pk.real * x.real - Pk.imag * x.imag).sum(1).T       # real products, as in the kernel
+    im = (Pk.real * x.imag + Pk.imag * x.real).sum(1).T
+    assert np.isinf(re).any() and np.isinf(im).any()
+    for g, e in ((got.real, re), (got.imag, im)):
+        fin = np.isfinite(e)
+        assert np.isinf(e[~fin]).all() and (g[~fin] == e[~fin]).all()
+        assert np.isfinite(g[fin]).all()
+
+
 def test_precode_group_beyond_32_bit_byte_offsets():
     """One group's precoder of 4 GiB and a little: antennas past 2^29 read their
     own entries (times 2: exact)."""
