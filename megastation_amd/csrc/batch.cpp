@@ -50,8 +50,7 @@ struct EqPlanChoice {
       c.kind = EqKind::Reg;
       return true;
     }
-    if (std::sscanf(s.c_str(), "wide MT=%u KS=%u chunks=%u", &c.MT, &c.KS, &c.chunks) == 3 &&
-        c.chunks >= 1) {
+    if (std::sscanf(s.c_str(), "wide MT=%u KS=%u chunks=%u", &c.MT, &c.KS, &c.chunks) == 3) {
       c.kind = EqKind::Wide;
       return true;
     }
@@ -483,13 +482,15 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
       return bail(MEGA_ERR_UNSUPPORTED, "no equalize plan for B=" + std::to_string(q.B));
     q.plan = cands[0];
     auto it = cache.find(q.key);
+    // a saved plan counts only as one of today's candidates: a line of an older
+    // candidate set or a damaged one is measured again, never run
     EqPlanChoice saved;
-    if (it != cache.end() && EqPlanChoice::parse(it->second, saved) &&
-        (saved.kind != EqKind::Wide ||
-         (q.B <= 256 && saved.MT == user_tiles(maxU) && saved.KS == (q.B <= 128 ? 4u : 8u)))) {
-      q.plan = saved;
-      tune[k] = false;
-    }
+    if (it != cache.end() && EqPlanChoice::parse(it->second, saved))
+      for (const auto& c : cands)
+        if (c.str() == saved.str()) {
+          q.plan = c;
+          tune[k] = false;
+        }
   }
   if ((e = build()) != hipSuccess) return hip_bail(e, "batch tables");
   if ((e = run_launches(b, b->stream, false)) != hipSuccess) return hip_bail(e, "batch warm-up");

@@ -104,6 +104,39 @@ WIDE_CELLS = [  # every wide tile plan: 1, 2 and 4 user tiles, 64-128 and 160-25
 ]
 
 
+@pytest.mark.parametrize("saved", [
+    "stream MT=2 waves/CU=12",          # the candidate set before the wide form
+    "wide MT=1 KS=4 chunks=4294967295",  # more chunks than 32-bit sums hold
+    "wide MT=1 KS=4 chunks=0", "wide MT=2 KS=4 chunks=1", "wide MT=1 KS=8 chunks=1",
+    "reg MT=1 KS=8",                    # holds 32 of the 128 antennas
+    "reg MT=0 KS=8", "stream MT=0 waves/CU=0"])
+def test_batch_measures_saved_plans_that_are_no_candidate(saved, tmp_path, monkeypatch):
+    """A line of a tune file that is not one of the class's candidate plans (a
+    128-antenna class of 16 users here) is not run: the class is timed again,
+    the new choice appended, and the next batch takes that one."""
+    print(f"case: batch saved plan {saved!r}", flush=True)
+    t = torch()
+    monkeypatch.setitem(globals(), "CELLS", [(16, 128, 60, 12, 4, "standalone")])
+    cells = _make_cells(seed=9)
+    path = tmp_path / "tune.txt"
+    path.write_text(f"B=128;16x60/12x2\t{saved}\n")
+    b = m.Batch(cells, tune_path=str(path))
+    assert "(cached)" not in b.plan()
+    b.run()
+    t.cuda.synchronize()
+    b.close()
+    c = cells[0]
+    w64, _, _ = oracle.zf(c["slot"].csi, 16, 128, 5, "f64")
+    for s in range(c["S"]):
+        llr64, x64 = oracle_symbol_f64(w64, c["slot"].y[s], 16, 128, 60, 12, 4, c["layout"])
+        check_symbol(host_u16(c["llr"]).reshape(2, 16, -1)[s], host_c64(c["xhat"]).reshape(2, 16, 60)[s],
+                     llr64, x64, 60, 12, 4, c["layout"])
+    assert len(path.read_text().splitlines()) == 2
+    b = m.Batch(cells, tune_path=str(path))
+    assert b.plan().count("(cached)") == 1
+    b.close()
+
+
 def test_batch_wide_plans_agree_for_every_chunk_count(tmp_path, monkeypatch):
     """The wide units' results do not depend on how a group's column tiles are
     cut into chunks (1, 2 or 5, forced through the plan file), and match FP64."""
