@@ -28,7 +28,11 @@
 // 490 -> 300; 1100 of Zc 144 585 -> 415.
 // Per check and row, exactly the operations of the CPU oracle in the same
 // order (round-to-nearest FP32 subtract, multiply and add, no contraction),
-// so the decoded bits and the final LLRs equal the oracle's.
+// so the bits decoded from finite LLRs equal the oracle's. Infinities are
+// carried as such. A NaN, of the input with either sign or of infinities that
+// cancel, counts as not negative, as in the oracle, and never as the minimum;
+// v_med3 then returns the smallest of its operands, so it also takes min2 down
+// to min1 (the tests hold the decoder to that, bit for bit).
 #include <hip/hip_runtime.h>
 
 #include <cstddef>

@@ -100,6 +100,68 @@ def test_more_code_blocks_than_cus_match_oracle(bg, zc, mb, half, n_cb):
     assert np.all(out[:, words:] == 0xFFFFFFFF)
 
 
+def _decode_numpy(llr, bg, zc, mb, iters, alpha):
+    """The layered schedule in numpy FP32 with the kernel's rule for NaN: not
+    negative, never the minimum, min2 down to min1 (llr [n][(kb + mb) * zc])."""
+    rs, col, shift = ldpc.tables(bg)
+    sh, n, f32 = shift[ldpc.set_index(zc)], len(llr), np.float32
+    L = llr.reshape(n, -1, zc).copy()
+    R = np.zeros((rs[mb], n, zc), f32)
+    for _ in range(iters):
+        for r in range(mb):
+            es = range(rs[r], rs[r + 1])
+            q = [np.roll(L[:, col[e]], -(sh[e] % zc), axis=1) - R[e] for e in es]
+            min1 = np.full((n, zc), np.inf, f32)
+            min2, at, par = min1.copy(), np.zeros((n, zc), int), np.zeros((n, zc), bool)
+            for i, x in enumerate(q):
+                a = np.abs(x)
+                at[a < min1] = i
+                min2 = np.where(np.isnan(a), min1, np.maximum(min1, np.fmin(min2, a)))
+                min1 = np.fmin(min1, a)
+                par ^= x < 0
+            for i, (e, x) in enumerate(zip(es, q)):
+                mag = f32(alpha) * np.where(at == i, min2, min1)
+                R[e] = np.where(par ^ (x < 0), -mag, mag)
+                L[:, col[e]] = np.roll(x + R[e], sh[e] % zc, axis=1)
+    bits = (L.reshape(n, -1)[:, :ldpc.KB[bg] * zc] < 0).astype(np.uint8)
+    pad = np.zeros((n, -bits.shape[1] % 32), np.uint8)
+    return np.packbits(np.hstack([bits, pad]), axis=1, bitorder="little").view(np.uint32)
+
+
+@pytest.mark.parametrize("bg,zc,mb,half,n_cb", [(1, 288, 46, True, 258), (1, 64, 46, False, 5),
+                                                (2, 384, 12, False, 257), (2, 15, 42, True, 5)])
+@pytest.mark.filterwarnings("ignore:invalid value")
+def test_infinite_and_nan_llrs(bg, zc, mb, half, n_cb):
+    """Infinities of both signs (some cancel within a row) and NaN of both
+    signs, one and two code blocks a workgroup: the bits of the same schedule in
+    numpy, which agrees with the oracle where everything is finite."""
+    print(f"case: ldpc non-finite bg={bg} zc={zc} mb={mb} half={half} n_cb={n_cb}", flush=True)
+    nv, words = (ldpc.KB[bg] + mb) * zc, (ldpc.KB[bg] * zc + 31) // 32
+    rng = np.random.default_rng(zc + 1)
+    dt, it, nan = ((np.float16, np.uint16, (0x7e00, 0xfe00)) if half else
+                   (np.float32, np.uint32, (0x7fc00000, 0xffc00000)))
+    finite = rng.standard_normal((5, nv)).astype(dt)
+    assert np.array_equal(_decode_numpy(finite.astype(np.float32), bg, zc, mb, 2, 0.8125),
+                          ldpc.decode(finite.astype(np.float32), bg, zc, mb, 2, 0.8125))
+    t = torch()
+    turn = np.arange(n_cb) % 5
+    for p_inf, p_nan in ((0.02, 0.0), (0.0, 0.002), (0.3, 0.05)):
+        llr = finite.copy()
+        u = rng.random(llr.shape)
+        inf = u < p_inf
+        llr[inf] = np.where(rng.random(inf.sum()) < 0.5, np.inf, -np.inf)
+        isnan = u > 1 - p_nan
+        llr.view(it)[isnan] = np.array(nan, it)[rng.integers(0, 2, isnan.sum())]
+        dev = t.from_numpy(llr.view(np.int16 if half else np.int32)[turn]).to("cuda:0")
+        for iters, alpha in ((1, 0.0), (3, 1.0)):  # 0 selects 0.8125
+            out = t.zeros(n_cb, words, dtype=t.int32, device="cuda:0")
+            m.ldpc_decode(dev.view(t.float16 if half else t.float32), out, base_graph=bg,
+                          lifting_size=zc, parity_nodes=mb, max_iterations=iters, num_cb=n_cb,
+                          llr_stride=nv, out_stride=words, normalization=alpha)
+            ref = _decode_numpy(llr.astype(np.float32), bg, zc, mb, iters, alpha or 0.8125)
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), ref[turn]), (p_inf, iters)
+
+
 def test_equalizer_llrs_decode_to_transmitted_bits():
     """64 x 16 cell, 1200 subcarriers, 16-QAM at -4 dB per antenna (about
     13 dB after ZF's array gain; the hard decisions of about 2 % of the coded
