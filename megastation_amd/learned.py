@@ -91,6 +91,19 @@ def gemm(A, sai, sak, B, sbk, sbj, M, N, K, *, bias=None, act=IDENTITY, Cf=None,
     _check(_L().mega_mlp_gemm(ctypes.byref(d), _stream(stream)))
 
 
+def _used_on(stream, *tensors):
+    """Tensors allocated on the current stream and used on `stream`: their memory
+    must not be handed out again before that stream's work is through."""
+    if stream is None:
+        return
+    import torch
+    h = getattr(stream, "cuda_stream", stream)
+    s = torch.cuda.ExternalStream(h) if h else torch.cuda.default_stream()
+    for t in tensors:
+        if t is not None:
+            t.record_stream(s)
+
+
 def n_features(U: int) -> int:
     return 2 * U * (U + 1)
 
@@ -154,6 +167,7 @@ class WarmStartNet:
             else:
                 z = torch.empty(M, n_out, device="cuda")
                 hb = None if last else torch.empty(M, n_out, dtype=torch.bfloat16, device="cuda")
+                _used_on(stream, z, hb)
             gemm(h, n_in, 1, self.wb[l], n_out, 1, M, n_out, n_in, bias=self.b[l],
                  act=IDENTITY if last else GELU, Cf=z, Cb=hb, stream=stream)
             zs.append(z)
@@ -191,6 +205,8 @@ class WarmStartNet:
             layers[l] = Layer(saved[l].data_ptr(), self.wb[l].data_ptr(), zs[l].data_ptr(), p[0],
                               p[1], gw[l].data_ptr(), gb[l].data_ptr(), p[2], n_in, n_out,
                               IDENTITY if l == 2 else GELU)
+        # the forward's tensors too: the next forward drops them
+        _used_on(stream, tmp, dout, *saved, *zs, *gw, *gb)
         _check(_L().mega_mlp_backward(layers, 3, M, _ptr(dout), _stream(stream)))
         self.grads = gw + gb
         return self.grads
@@ -206,6 +222,7 @@ class WarmStartNet:
     def mse_grad(self, out, target, stream=None):
         import torch
         d = torch.empty_like(out)
+        _used_on(stream, d)
         _check(_L().mega_mlp_mse_grad(_ptr(out), _ptr(target), _ptr(d), out.numel(),
                                       out.shape[0], _stream(stream)))
         return d

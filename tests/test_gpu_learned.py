@@ -110,6 +110,38 @@ def test_col_sum_is_four_running_sums(M, N):
     assert np.array_equal(db.cpu().numpy(), (p[0] + p[1]) + (p[2] + p[3]))
 
 
+def test_training_step_on_another_stream_keeps_its_buffers():
+    """A whole step on a side stream that has not begun when the calls return:
+    none of the memory it uses may be handed out meanwhile. Tensors filled on the
+    current stream from all the allocator would hand out keep their values, and
+    the step's weights are those of the same step on the current stream."""
+    print("case: training step on a side stream", flush=True)
+    t = torch()
+    M, out = 600, []
+    x = t.randn(M, learned.n_features(16), device="cuda").to(t.bfloat16)
+    y = t.randn(M, learned.n_outputs(16), device="cuda")
+    for side in (None, t.cuda.Stream()):
+        net = learned.WarmStartNet(16, seed=3)
+        t.cuda.synchronize()
+        if side is not None:
+            with t.cuda.stream(side):
+                t.cuda._sleep(20_000_000)
+        d = net.mse_grad(net.forward(x, keep=True, stream=side), y, stream=side)
+        net.backward(d, stream=side)
+        net.adam(stream=side)
+        net._saved = net.grads = d = None
+        if side is not None:
+            held, reserved = [], t.cuda.memory_reserved()
+            while t.cuda.memory_reserved() == reserved and len(held) < 4096:
+                held.append(t.full((1 << 20,), 7, dtype=t.uint8, device="cuda"))
+                held.append(t.full((256,), 7, dtype=t.uint8, device="cuda"))
+            assert not side.query()  # the step is still to come
+        t.cuda.synchronize()
+        out.append([p.clone() for p in net.params])
+    assert all(bool((h == 7).all()) for h in held)
+    assert all(t.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize("sizes", [(1,), (257, 0, 256, 1000), (3, 5, 70, 1, 0, 2, 300, 9, 11, 4)])
 def test_adam_group_equals_single_tensors(sizes):
     """Several tensors a launch (empty ones, more than eight) against a call for
