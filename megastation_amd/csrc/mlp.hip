@@ -615,7 +615,7 @@ hipError_t mlp_adam(const mega_mlp_tensor* t, uint32_t count, float lr, float b1
       if (t[i].n == 0) continue;
       const uint64_t nb = (t[i].n + kAdamThreads - 1) / kAdamThreads;
       if (nb > 0x7fffffffu) return hipErrorInvalidConfiguration;
-      if (k && nb > 0x7fffffffu - blocks) break;  // the next launch's
+      if (k && nb > 0xffffffffu / kAdamThreads - blocks) break;  // a launch's threads: 32 bits
       a.t[k] = t[i];
       a.end[k++] = blocks += (uint32_t)nb;
     }

@@ -110,6 +110,28 @@ def test_col_sum_is_four_running_sums(M, N):
     assert np.array_equal(db.cpu().numpy(), (p[0] + p[1]) + (p[2] + p[3]))
 
 
+def test_adam_group_beyond_the_threads_of_a_launch():
+    """Two tensors of 2^31 weights and a few: more threads than a launch has, so
+    a launch each. (w, g, m and v of a tensor are one buffer, which the kernel's
+    order of reads and writes allows, to keep the test small.)"""
+    n = 2**31 + 300
+    print(f"case: adam group 2 x {n}", flush=True)
+    t = torch()
+    L = learned._L()
+    args = (1e-3, 0.9, 0.999, 1e-8, 1, m._stream(None))
+    group, single = ([t.full((n,), x, device="cuda") for x in (0.5, 0.25)] for _ in range(2))
+    for b in group + single:
+        b[-1] = 2.0
+    for b in single:
+        m._check(L.mega_mlp_adam(m._ptr(b), None, m._ptr(b), m._ptr(b), m._ptr(b), n, *args))
+    ts = (learned.Tensor * 2)(*[
+        learned.Tensor(b.data_ptr(), None, b.data_ptr(), b.data_ptr(), b.data_ptr(), n)
+        for b in group])
+    m._check(L.mega_mlp_adam_group(ts, 2, *args))
+    for a, b in zip(group, single):
+        assert t.equal(a, b) and float(a[0]) != float(a[-1]) and float(a[0]) not in (0.5, 0.25)
+
+
 def test_training_step_on_another_stream_keeps_its_buffers():
     """A whole step on a side stream that has not begun when the calls return:
     none of the memory it uses may be handed out meanwhile. Tensors filled on the
