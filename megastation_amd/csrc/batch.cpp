@@ -30,11 +30,13 @@ struct ZfClass {
 
 struct EqPlanChoice {
   EqKind kind = EqKind::Stream;
-  uint32_t MT = 4, KS = 0, waves_per_cu = 12, chunks = 1;
+  uint32_t MT = 4, KS = 0, waves_per_cu = 12;
+  uint32_t chunks = 0, tiles = 0;  // wide: a group's chunks, or a chunk's column tiles
   std::string str() const {
     std::ostringstream o;
     if (kind == EqKind::Wide)
-      o << "wide MT=" << MT << " KS=" << KS << " chunks=" << chunks;
+      o << "wide MT=" << MT << " KS=" << KS << (chunks ? " chunks=" : " tiles=")
+        << (chunks ? chunks : tiles);
     else if (kind == EqKind::Stream)
       o << "stream MT=" << MT << " waves/CU=" << waves_per_cu;
     else
@@ -51,6 +53,11 @@ struct EqPlanChoice {
       return true;
     }
     if (std::sscanf(s.c_str(), "wide MT=%u KS=%u chunks=%u", &c.MT, &c.KS, &c.chunks) == 3) {
+      c.kind = EqKind::Wide;
+      return true;
+    }
+    c.chunks = 0;
+    if (std::sscanf(s.c_str(), "wide MT=%u KS=%u tiles=%u", &c.MT, &c.KS, &c.tiles) == 3) {
       c.kind = EqKind::Wide;
       return true;
     }
@@ -77,7 +84,8 @@ uint32_t eq_units(EqParams& p, const EqPlanChoice& c) {
     return p.G * p.col_tiles * p.nmg;
   }
   if (c.kind == EqKind::Wide) {
-    p.tiles_per_wg = (p.col_tiles + c.chunks - 1) / c.chunks;
+    p.tiles_per_wg =
+        c.chunks ? (p.col_tiles + c.chunks - 1) / c.chunks : std::min(c.tiles, p.col_tiles);
     p.chunks = (p.col_tiles + p.tiles_per_wg - 1) / p.tiles_per_wg;
     return p.G * p.chunks;
   }
@@ -92,22 +100,53 @@ uint32_t eq_units(EqParams& p, const EqPlanChoice& c) {
 // 16-user tiles of a class (the wide form's).
 uint32_t user_tiles(uint32_t U) { return U <= 16 ? 1 : U <= 32 ? 2 : 4; }
 
-std::vector<EqPlanChoice> eq_candidates(uint32_t B, uint32_t maxU) {
+// Workgroups of the wide form (512 threads) that a launch's 32-bit thread count holds.
+constexpr uint64_t kMaxWideUnits = 0xffffffffu / 512;
+
+// Candidate plans of a class: cells of one antenna count, up to maxU users.
+std::vector<EqPlanChoice> eq_candidates(uint32_t B, uint32_t maxU,
+                                        const std::vector<EqParams>& cells) {
   std::vector<EqPlanChoice> v;
   // The wide form up to 256 antennas, W_g once per chunk of a group's column
   // tiles: one or two chunks where the batch fills the chip, five for short
   // batches. Beyond, streamed W (256 x 64, 1667 groups: 385 us against 516
   // streamed; 128 x 32, 1655 groups: 110 against 145).
   if (B % 32 == 0 && B > 32 && B <= 256) {
+    EqPlanChoice c;
+    c.kind = EqKind::Wide;
+    c.MT = user_tiles(maxU);
+    c.KS = B <= 128 ? 4 : 8;
+    std::vector<EqPlanChoice> cuts;
     for (uint32_t n : {1u, 2u, 5u}) {
-      EqPlanChoice c;
-      c.kind = EqKind::Wide;
-      c.MT = user_tiles(maxU);
-      c.KS = B <= 128 ? 4 : 8;
       c.chunks = n;
-      v.push_back(c);
+      cuts.push_back(c);
     }
-  } else if (B % 32 == 0) {
+    // Groups of so many columns that a fifth is more than a CU's share of the
+    // class: chunks of half that share and of all of it (a batch of one group
+    // of 3276 subcarriers x 13 symbols, 256 x 32: 68 us; five chunks 1365,
+    // streamed 278)
+    uint64_t total = 0, most = 0;
+    for (const EqParams& p : cells) {
+      total += (uint64_t)p.G * p.col_tiles;
+      most = std::max<uint64_t>(most, p.col_tiles);
+    }
+    c.chunks = 0;
+    for (uint32_t wgs : {2 * kCUs, kCUs}) {
+      const uint64_t share = (total + wgs - 1) / wgs;
+      if (share >= (most + 4) / 5) continue;
+      c.tiles = (uint32_t)share;
+      cuts.push_back(c);
+    }
+    for (const EqPlanChoice& c : cuts) {
+      uint64_t units = 0;
+      for (EqParams p : cells) {
+        eq_units(p, c);
+        units += (uint64_t)p.G * p.chunks;
+      }
+      if (units <= kMaxWideUnits) v.push_back(c);
+    }
+  }
+  if (B % 32 == 0 && v.empty()) {
     for (uint32_t MT : {1u, 2u, 4u}) {
       if (MT > 1 && 8 * (MT / 2) >= maxU) continue;  // a smaller tile already covers all users
       for (uint32_t w : {8u, 12u, 16u}) {
@@ -471,13 +510,20 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
   // Every class starts on its first candidate (or the cached choice); one run
   // with those computes W, then each class without a cached choice times its
   // candidates alone on the batch's own buffers and keeps the fastest.
+  auto candidates = [&](const EqClass& q) {
+    uint32_t maxU = 0;
+    std::vector<EqParams> ps;
+    for (uint32_t i : q.cells) {
+      maxU = std::max(maxU, b->eqp[i].U);
+      ps.push_back(b->eqp[i]);
+    }
+    return eq_candidates(q.B, maxU, ps);
+  };
   auto cache = read_cache(tune_path);
   std::vector<bool> tune(b->eq.size(), true);
   for (size_t k = 0; k < b->eq.size(); ++k) {
     EqClass& q = b->eq[k];
-    uint32_t maxU = 0;
-    for (uint32_t i : q.cells) maxU = std::max(maxU, b->eqp[i].U);
-    const auto cands = eq_candidates(q.B, maxU);
+    const auto cands = candidates(q);
     if (cands.empty())
       return bail(MEGA_ERR_UNSUPPORTED, "no equalize plan for B=" + std::to_string(q.B));
     q.plan = cands[0];
@@ -502,11 +548,9 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
       tune_log << "  " << q.key << ": " << q.plan.str() << " (cached)\n";
       continue;
     }
-    uint32_t maxU = 0;
-    for (uint32_t i : q.cells) maxU = std::max(maxU, b->eqp[i].U);
     float best = 1e30f;
     EqPlanChoice best_c = q.plan;
-    for (const auto& c : eq_candidates(q.B, maxU)) {
+    for (const auto& c : candidates(q)) {
       q.plan = c;
       if ((e = build()) != hipSuccess) return hip_bail(e, "batch tables");
       const EqClassLaunch L = b->eq_launch[k];

@@ -104,6 +104,30 @@ WIDE_CELLS = [  # every wide tile plan: 1, 2 and 4 user tiles, 64-128 and 160-25
 ]
 
 
+@pytest.mark.parametrize("cell", [
+    (32, 256, 600, 600, 6, "standalone"), (8, 128, 601, 600, 4, "standalone"),
+    (40, 64, 700, 300, 2, "ldpc")])
+def test_batch_cuts_few_wide_groups_into_many_chunks(cell, tmp_path, monkeypatch):
+    """One to three groups of hundreds of column tiles (one of them a single
+    subcarrier): the plan cuts them into enough units for the chip, where five
+    chunks a group would leave most of it idle."""
+    print(f"case: batch few groups {cell}", flush=True)
+    t = torch()
+    monkeypatch.setitem(globals(), "CELLS", [cell])
+    U, B, N, sg, Q, _ = cell
+    c, = _make_cells(seed=11, S=7)
+    b = m.Batch([c], tune_path=str(tmp_path / "tune.txt"))
+    assert "tiles=" in b.plan(), b.plan()
+    b.run()
+    t.cuda.synchronize()
+    b.close()
+    w64, _, _ = oracle.zf(c["slot"].csi, U, B, (N + sg - 1) // sg, "f64")
+    for s in range(7):
+        llr64, x64 = oracle_symbol_f64(w64, c["slot"].y[s], U, B, N, sg, Q, c["layout"])
+        check_symbol(host_u16(c["llr"]).reshape(7, U, -1)[s], host_c64(c["xhat"]).reshape(7, U, N)[s],
+                     llr64, x64, N, sg, Q, c["layout"])
+
+
 @pytest.mark.parametrize("saved", [
     "stream MT=2 waves/CU=12",          # the candidate set before the wide form
     "wide MT=1 KS=4 chunks=4294967295",  # more chunks than 32-bit sums hold
