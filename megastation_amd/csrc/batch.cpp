@@ -74,6 +74,15 @@ struct EqClass {
 
 constexpr uint32_t kCUs = 256;
 
+// Column tiles up to which the cells of one antenna count are one class of the
+// widest cell's user tiles, its pad users' products being cheaper than a launch
+// of each width: two a CU, and 32 up to 64 antennas, which leave half of the
+// wide form's waves idle. Two cells of 4 and 20 users, us a batch apart and as
+// one: 96 antennas, 400 tiles 36.9 / 35.1, 12800 99 / 105; 64 antennas, 3200
+// tiles 47.5 / 44.1, 6400 65.4 / 62.9, 12800 88 / 96. (20 and 40 x 64, 3200 tiles
+// 77.3 / 69.1, where one streamed launch had taken 76.9.)
+constexpr uint32_t few_tiles(uint32_t B) { return B <= 64 ? 32 * kCUs : 2 * kCUs; }
+
 // The tile plan's per-cell fields and unit count.
 uint32_t eq_units(EqParams& p, const EqPlanChoice& c) {
   if (c.kind == EqKind::Stream) {
@@ -215,8 +224,13 @@ struct TableBuilder {
 };
 
 hipError_t run_launches(mega_batch* b, hipStream_t st, bool parallel) {
-  hipError_t e = launch_reset_counters(b->counters, b->ncounters, st);
-  if (e != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  // Only the streamed form counts (a launch, 2 us, less without it); but a graph
+  // of two branches starts from one node: with two roots three cells of 5 groups
+  // took 58 us instead of 49
+  bool count = parallel;
+  for (auto& L : b->eq_launch) count |= L.kind == EqKind::Stream;
+  if (count && (e = launch_reset_counters(b->counters, b->ncounters, st)) != hipSuccess) return e;
   // ZF classes: the widest on the side stream when parallel
   if (parallel && b->zf_launch.size() > 1) {
     if ((e = hipEventRecord(b->fork, st)) != hipSuccess) return e;
@@ -367,9 +381,16 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
   }
   {
     std::map<std::pair<uint32_t, uint32_t>, EqClass> byB;
+    std::map<uint32_t, std::pair<uint64_t, uint32_t>> work;  // B: tiles, user tiles
+    for (const EqParams& p : b->eqp) {
+      auto& w = work[p.B];
+      w.first += (uint64_t)p.G * p.col_tiles;
+      w.second = std::max(w.second, user_tiles(p.U));
+    }
     for (uint32_t i = 0; i < num_cells; ++i) {
-      EqClass& c = byB[{b->eqp[i].B, user_tiles(b->eqp[i].U)}];
-      c.B = b->eqp[i].B;
+      const uint32_t B = b->eqp[i].B, ut = user_tiles(b->eqp[i].U);
+      EqClass& c = byB[{B, work[B].first <= few_tiles(B) ? work[B].second : ut}];
+      c.B = B;
       c.cells.push_back(i);
     }
     for (auto& kv : byB) {
@@ -555,7 +576,8 @@ int mega_batch_create(const mega_cell_desc* cells, uint32_t num_cells, const cha
       if ((e = build()) != hipSuccess) return hip_bail(e, "batch tables");
       const EqClassLaunch L = b->eq_launch[k];
       const float ms = time_ms(b->stream, 4, [&]() {
-        hipError_t r = launch_reset_counters(L.counters, 8, b->stream);
+        hipError_t r = L.kind == EqKind::Stream ? launch_reset_counters(L.counters, 8, b->stream)
+                                                : hipSuccess;
         return r == hipSuccess ? launch_eq_class(L, b->stream) : r;
       }, e);
       if (e != hipSuccess) return hip_bail(e, "batch tuning");

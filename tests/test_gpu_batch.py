@@ -128,6 +128,50 @@ def test_batch_cuts_few_wide_groups_into_many_chunks(cell, tmp_path, monkeypatch
                      llr64, x64, N, sg, Q, c["layout"])
 
 
+def test_batch_small_cells_of_one_antenna_count_share_a_class(monkeypatch, tmp_path):
+    """Few column tiles: 4 to 64 users of 64 (and of 128) antennas are one equalize
+    class, padded to its widest cell's user tiles, with the bits of each cell alone."""
+    print("case: batch merged classes", flush=True)
+    t = torch()
+    monkeypatch.setitem(globals(), "CELLS", [
+        (4, 64, 60, 12, 2, "standalone"), (20, 64, 50, 12, 6, "ldpc"), (40, 64, 28, 16, 4, "standalone"),
+        (16, 128, 60, 12, 8, "standalone"), (64, 128, 30, 12, 2, "standalone"),
+        (17, 128, 24, 8, 4, "standalone")])
+    cells = _make_cells(seed=13, S=3)
+    outs = []
+    for alone in (False, True):
+        for c in cells:
+            c["llr"].fill_(SENTINEL)
+        for k, part in enumerate([[c] for c in cells] if alone else [cells]):
+            # the wide form in both (a 64-antenna cell alone may be timed faster
+            # with W in one wave's registers, whose sums differ)
+            path = tmp_path / f"tune{alone}{k}.txt"
+            m.Batch(part, tune_path=str(path)).close()
+            keys = [line.split("\t")[0] for line in path.read_text().splitlines()]
+            assert len(keys) == (1 if alone else 2)
+            mt = {key: max(int(x.split("x")[0]) for x in key.split(";")[1:]) for key in keys}
+            path.write_text("".join(
+                f"{key}\twide MT={1 if u <= 16 else 2 if u <= 32 else 4} KS=4 chunks=2\n"
+                for key, u in mt.items()))
+            b = m.Batch(part, tune_path=str(path))
+            assert b.plan().count("(cached)") == len(keys)
+            b.run()
+            t.cuda.synchronize()
+            b.close()
+        outs.append([(host_u16(c["llr"]).copy(), host_c64(c["xhat"]).copy()) for c in cells])
+    for (l0, x0), (l1, x1) in zip(*outs):
+        assert np.array_equal(l0, l1) and np.array_equal(x0, x1) and np.abs(x0).max() > 0
+
+
+def test_batch_wide_plans_of_every_user_tile_count(tmp_path, monkeypatch):
+    """As below, each antenna count with cells of one width."""
+    monkeypatch.setitem(globals(), "WIDE_CELLS", [
+        (16, 96, 204, 12, 2, "standalone"), (8, 160, 150, 16, 8, "standalone"),
+        (24, 224, 60, 12, 4, "standalone"), (17, 64, 100, 16, 4, "ldpc"),
+        (33, 128, 77, 8, 6, "standalone"), (50, 192, 41, 12, 8, "standalone")])
+    test_batch_wide_plans_agree_for_every_chunk_count(tmp_path, monkeypatch)
+
+
 @pytest.mark.parametrize("saved", [
     "stream MT=2 waves/CU=12",          # the candidate set before the wide form
     "wide MT=1 KS=4 chunks=4294967295",  # more chunks than 32-bit sums hold
