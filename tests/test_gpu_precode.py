@@ -99,6 +99,34 @@ def test_precode_ranges_match_fp64(B, U, N, sg, row, start, S):
     assert (np.abs(got - exp) <= 4 * U * 2.0 ** -23 * mag + 1e-30).all()
 
 
+@pytest.mark.parametrize("B,U,N,sg,S", [
+    (256, 3, 3276, 12, 13), (300, 7, 1650, 12, 13), (256, 13, 3276, 12, 13),  # tiles dealt round
+    (300, 21, 3276, 12, 13),                                                  # a group a wave
+    (160, 30, 3276, 12, 13), (200, 9, 3277, 12, 13), (96, 45, 3276, 12, 5),   # ranges of groups
+    (128, 10, 3280, 16, 14), (70, 61, 4000, 9, 14),                           # equal ranges
+])
+def test_precode_divisions_of_the_work_match_fp64(B, U, N, sg, S):
+    """Every way to divide a full slot's tiles and antenna blocks among waves,
+    with the bound of the test above."""
+    print(f"case: precode division B={B} U={U} N={N} sg={sg} S={S}", flush=True)
+    t = torch()
+    gen = t.Generator(device="cuda").manual_seed(B + U)
+    G = N // sg
+    P = t.randn(-(-N // sg), U, B, dtype=t.complex64, device="cuda", generator=gen)
+    ue = t.randn(S, U, N, dtype=t.complex64, device="cuda", generator=gen)
+    out = t.full((S, B, N + 3), complex(SENT), dtype=t.complex64, device="cuda")
+    half = (N + 3) // 2
+    m.precode(P, ue, out, num_bs=B, num_ue=U, num_sc=N, sc_group=sg, bs_stride=N + 3,
+              bs_start=N + 3 - half, num_syms=S)  # the columns as they are
+    A = P[:G].transpose(1, 2).to(t.complex128).contiguous()                  # [G][B][U]
+    X = ue[:, :, :G * sg].reshape(S, U, G, sg).permute(2, 1, 0, 3).reshape(G, U, S * sg)
+    X = X.to(t.complex128).contiguous()
+    unfold = lambda y: y.reshape(G, B, S, sg).permute(2, 1, 0, 3).reshape(S, B, G * sg)
+    err = (out[:, :, :G * sg] - unfold(A @ X)).abs()
+    assert bool((err <= 4 * U * 2.0 ** -23 * unfold(A.abs() @ X.abs())).all())
+    assert bool((out[:, :, G * sg:] == complex(SENT)).all())
+
+
 @pytest.mark.parametrize("U,B", [(2, 40), (6, 200), (17, 64), (18, 130), (34, 70)])
 def test_precode_infinities_of_the_last_user(U, B):
     """Users are padded to whole steps: an infinite entry or symbol of the last
