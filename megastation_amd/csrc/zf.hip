@@ -88,35 +88,46 @@ hipError_t launch_zf_ut(uint32_t U, uint32_t B, uint32_t batch, const float2* in
 // bound by the latency of its one pass: all loads of a thread are in flight
 // together, the values wait for the maximum in LDS (rows of an odd pitch, so
 // neither the column writes nor the row reads conflict) and leave as whole
-// antenna rows. A group beyond the LDS tile takes the maximum first and reads
-// its antennas a second time, a tile at a time (bt = 0, a user count no tile
-// holds: stored straight). Storing straight from the
-// column order scattered every 8 bytes to a line of its own: 33.8 us against
-// 14.2 at 273 groups of 256 x 32 (36 MB).
+// antenna rows; eight entries a thread, so that small groups share a CU (15000
+// groups of 64 x 16: 113 us with 1024 threads each, 37 now). A group beyond the
+// LDS tile takes the maximum first and reads its antennas a second time, a tile
+// at a time (bt = 0, a user count no tile holds: stored straight). Storing
+// straight from the column order scattered every 8 bytes to a line of its own:
+// 33.8 us against 14.2 at 273 groups of 256 x 32 (36 MB; back to back 24.0 and
+// 11.5).
+__device__ __forceinline__ float square(float2 v) {  // |v|^2, one order for both kernels
+  return __builtin_fmaf(v.x, v.x, v.y * v.y);
+}
 constexpr uint32_t kScaleLds = 16384 + 128;  // float2 of the tile
 __global__ __launch_bounds__(1024) void scale_absmax_kernel(
     const float2* __restrict__ in, float2* __restrict__ out, uint32_t U,
-    uint32_t B, uint32_t batch, uint32_t bt, uint32_t pitch) {
+    uint32_t B, uint32_t batch, uint32_t bt, uint32_t pitch, uint32_t u_inv) {
   __shared__ float sMax[1024 / 64];
   extern __shared__ float sDyn[];
   float2* tile = reinterpret_cast<float2*>(sDyn);  // [U][pitch], bt antennas
   const uint32_t n = U * B, nt = blockDim.x;
   const bool whole = bt >= B;
+  auto put = [&](uint32_t e, float2 v) {  // antenna e / U of the tile, user e % U
+    const uint32_t b = div_by(e, U, u_inv);
+    tile[(e - b * U) * pitch + b] = v;
+  };
   for (uint32_t g = blockIdx.x; g < batch; g += gridDim.x) {
     const float2* x = in + (uint64_t)g * n;
     float2* o = out + (uint64_t)g * n;
     float m = 0.f;
-    for (uint32_t e0 = threadIdx.x; e0 < n; e0 += 8 * nt) {
-      float2 v[8];
+    constexpr int R = 8;  // loads in flight
+    for (uint32_t e0 = threadIdx.x; e0 < n; e0 += R * nt) {
+      float2 v[R];
 #pragma unroll
-      for (int r = 0; r < 8; ++r) v[r] = x[min(e0 + r * nt, n - 1)];
+      for (int r = 0; r < R; ++r) v[r] = x[min(e0 + r * nt, n - 1)];
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
+      for (int r = 0; r < R; ++r) {
         const uint32_t e = e0 + r * nt;
-        m = fmaxf(m, sqrtf(v[r].x * v[r].x + v[r].y * v[r].y));
-        if (whole && e < n) tile[(e % U) * pitch + e / U] = v[r];
+        m = fmaxf(m, square(v[r]));
+        if (whole && e < n) put(e, v[r]);
       }
     }
+    m = sqrtf(m);  // of the largest square: rounding keeps the order
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0) sMax[threadIdx.x >> 6] = m;
@@ -133,17 +144,47 @@ __global__ __launch_bounds__(1024) void scale_absmax_kernel(
       const uint32_t nb = min(bt, B - b0);
       if (!whole) {
         __syncthreads();  // the previous tile is out
-        for (uint32_t e = threadIdx.x; e < U * nb; e += nt)
-          tile[(e % U) * pitch + e / U] = x[(uint64_t)b0 * U + e];
+        for (uint32_t e = threadIdx.x; e < U * nb; e += nt) put(e, x[(uint64_t)b0 * U + e]);
         __syncthreads();
       }
+      const uint32_t nb_inv = div_inv(nb);
       for (uint32_t e = threadIdx.x; e < U * nb; e += nt) {
-        const uint32_t u = e / nb, b = e % nb;
+        const uint32_t u = div_by(e, nb, nb_inv), b = e - u * nb;
         const float2 v = tile[u * pitch + b];
         o[(uint64_t)u * B + b0 + b] = make_float2(v.x * s - v.y * 0.f, v.x * 0.f + v.y * s);
       }
     }
     __syncthreads();
+  }
+}
+
+// Groups of up to 64 R entries, a wave each, values in its registers: nothing
+// to gain from the tile, whose two barriers and LDS round trip cost more than
+// the group (40000 groups of 8 x 4: 21.4 us through it, 9.5 here; 12.9 stored
+// straight by a workgroup each).
+template <int R>
+__global__ __launch_bounds__(256) void scale_absmax_small(
+    const float2* __restrict__ in, float2* __restrict__ out, uint32_t U, uint32_t B,
+    uint32_t batch, uint32_t u_inv) {
+  const uint32_t n = U * B, lane = threadIdx.x & 63;
+  const uint64_t step = (uint64_t)gridDim.x * 4;
+  for (uint64_t g = blockIdx.x * 4ull + threadIdx.x / 64; g < batch; g += step) {
+    float2 v[R];
+    float m = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = in[g * n + min(lane + 64 * r, n - 1)];
+#pragma unroll
+    for (int r = 0; r < R; ++r) m = fmaxf(m, square(v[r]));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    const float s = 1.0f / sqrtf(m);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const uint32_t e = lane + 64 * r, b = div_by(e, U, u_inv);
+      if (e < n)
+        out[g * n + (e - b * U) * B + b] =
+            make_float2(v[r].x * s - v[r].y * 0.f, v[r].x * 0.f + v[r].y * s);
+    }
   }
 }
 
@@ -182,12 +223,18 @@ hipError_t launch_scale_absmax(uint32_t U, uint32_t B, uint32_t batch,
                                hipStream_t st) {
   if (batch == 0) return hipSuccess;
   const uint64_t n = (uint64_t)U * B;
-  const uint32_t threads = n >= 1024 ? 1024 : ((uint32_t)n + 63) / 64 * 64;
+  if (n <= 256) {
+    const auto fn = n <= 64 ? &scale_absmax_small<1> : &scale_absmax_small<4>;
+    hipLaunchKernelGGL(fn, dim3(std::min(batch / 4 + (batch % 4 > 0), 65535u)), dim3(256), 0, st,
+                       in, out, U, B, batch, div_inv(U));
+    return hipGetLastError();
+  }
   const uint32_t blocks = batch < 65536 ? batch : 65535;
-  // antennas per LDS tile: the whole group where it fits
+  // antennas per LDS tile: the whole group where it fits, else 8192 entries and
+  // at least 64 antennas
   uint32_t bt = B;
   if ((uint64_t)U * (B | 1) > kScaleLds) {
-    bt = std::min(64u, kScaleLds / U);
+    bt = std::min(std::max(64u, 8192 / U), kScaleLds / U);
     bt -= bt > 0 && bt % 2 == 0;  // an odd pitch within the tile
   }
   const uint32_t pitch = bt | 1;
@@ -198,8 +245,9 @@ hipError_t launch_scale_absmax(uint32_t U, uint32_t B, uint32_t batch,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
+  const uint32_t threads = (uint32_t)std::min<uint64_t>(1024, (n + 511) / 512 * 64);
   hipLaunchKernelGGL(scale_absmax_kernel, dim3(blocks), dim3(threads), lds, st, in, out, U, B,
-                     batch, bt, pitch);
+                     batch, bt, pitch, div_inv(U));
   return hipGetLastError();
 }
 

@@ -172,6 +172,34 @@ def test_precode_group_beyond_32_bit_byte_offsets():
         assert t.equal(out[lo:lo + 2**26], P[lo:lo + 2**26]), lo
 
 
+@pytest.mark.parametrize("U,B,G", [
+    (8, 8, 5), (5, 13, 7), (2, 1, 300000), (16, 16, 9), (1, 250, 3),  # a wave a group
+    (1, 257, 3), (3, 171, 2), (16, 64, 70000),                        # one LDS tile
+    (4, 5000, 2), (16, 1100, 2), (3, 11011, 2), (130, 128, 2)])       # several
+def test_precoder_normalisation_of_small_and_tall_groups(U, B, G):
+    """As below, against torch in 64 bits; and groups of zeros, of an infinity and
+    with a NaN (which the maximum passes over) give what the expression gives."""
+    print(f"case: precoder normalisation U={U} B={B} G={G}", flush=True)
+    t = torch()
+    W = t.randn(G, B, U, dtype=t.complex64, device="cuda",
+                generator=t.Generator(device="cuda").manual_seed(U + B))
+    W[1] = 0
+    W[0, B // 2, U // 2] = complex(np.inf, 1)
+    if G > 2 and U * B > 2:
+        W[2, B - 1, U - 1] = complex(np.nan, 2)
+    P = t.zeros(G, U, B, dtype=t.complex64, device="cuda")
+    m.Beamform.beamform_downlink(W, P, U, B, G)
+    w = W.to(t.complex128)
+    mag = t.nan_to_num(w.abs(), nan=0.0, posinf=np.inf).amax((1, 2), keepdim=True)
+    for got, part in ((P.real, w.real), (P.imag, w.imag)):
+        e = (part / mag).transpose(1, 2)
+        assert bool(((got - e).abs()[3:] < 4 * 2.0 ** -23).all())
+        for g in range(min(3, G)):
+            fin = t.isfinite(e[g]) & t.isfinite(w[g].real.T) & t.isfinite(w[g].imag.T)
+            assert bool(((got[g] - e[g]).abs()[fin] < 4 * 2.0 ** -23).all())
+            assert not bool(t.isfinite(got[g][~fin]).any())
+
+
 @pytest.mark.parametrize("U,B,G", [(1, 1, 3), (32, 256, 5), (64, 256, 2), (128, 300, 2), (100, 1, 4),
                                    (17000, 2, 1)])
 def test_precoder_normalisation_shapes(U, B, G):
