@@ -431,6 +431,31 @@ __global__ __launch_bounds__(CS_THREADS) void col_sum(const float* __restrict__ 
   if (w == 0 && j < N) db[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
 }
 
+// The same sums straight from memory, 64 columns a workgroup and a wave for each
+// i % 4, eight rows in flight: for few rows, where col_sum's 1024 threads have
+// little to bring, and for so many columns that these workgroups fill the chip
+// too (mlp_col_sum).
+__global__ __launch_bounds__(256) void col_sum_few(const float* __restrict__ dZ,
+                                                   float* __restrict__ db, uint32_t M,
+                                                   uint32_t N) {
+  __shared__ float part[4][64];
+  const uint32_t c = threadIdx.x & 63, w = threadIdx.x >> 6, j = blockIdx.x * 64 + c;
+  const float* p = dZ + min(j, N - 1);
+  float s = 0.f;
+  uint32_t i = w;
+  for (; i + 28 < M; i += 32) {
+    float x[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = p[(uint64_t)(i + 4 * q) * N];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s += x[q];
+  }
+  for (; i < M; i += 4) s += p[(uint64_t)i * N];
+  part[w][c] = s;
+  __syncthreads();
+  if (w == 0 && j < N) db[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+}
+
 // Gradient (y - t)/M of the MSE loss 0.5/M * sum (y - t)^2.
 __global__ void mse_grad(const float* __restrict__ Y, const float* __restrict__ T,
                          float* __restrict__ dY, uint64_t n, float inv_m) {
@@ -587,7 +612,15 @@ hipError_t mlp_act_backward(const float* dY, const float* Z, __bf16* dZ, float* 
 
 hipError_t mlp_col_sum(const float* dZ, float* db, uint32_t M, uint32_t N, hipStream_t st) {
   if (N == 0) return hipSuccess;
-  hipLaunchKernelGGL(col_sum, dim3(blocks_for(N, CS_COLS)), dim3(CS_THREADS), 0, st, dZ, db, M, N);
+  // us, through LDS / straight (with one row in flight): 8 x 512
+  // 3.6 / 2.8, 256 x 2112 4.1 / 3.6 (8.8), 512 x 2112 4.5 / 4.7, 1024 x 2112 5.4 /
+  // 7.2 (28.6), 1024 x 8000 14.5 / 13.9, 4096 x 8000 44.7 / 48.7, 4096 x 20000 95 /
+  // 83 (416), 8 x 100000 26 / 3.0
+  if (M <= 384 || N >= 16384)
+    hipLaunchKernelGGL(col_sum_few, dim3(blocks_for(N, 64)), dim3(256), 0, st, dZ, db, M, N);
+  else
+    hipLaunchKernelGGL(col_sum, dim3(blocks_for(N, CS_COLS)), dim3(CS_THREADS), 0, st, dZ, db, M,
+                       N);
   return hipGetLastError();
 }
 

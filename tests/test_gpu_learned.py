@@ -96,6 +96,12 @@ def test_gemm_of_an_empty_sum_is_its_epilogue(M, N):
     assert t.equal(Cb, bias.to(t.bfloat16).expand(M, N))
 
 
+@pytest.mark.parametrize("M,N", [(1, 64), (31, 65), (32, 100), (37, 16400), (384, 63),
+                                 (385, 63), (500, 16384), (500, 16383)])
+def test_col_sum_of_few_rows_or_many_columns(M, N):
+    test_col_sum_is_four_running_sums(M, N)
+
+
 @pytest.mark.parametrize("M,N", [(1, 5), (3, 16), (1024, 17), (1025, 40), (2111, 33)])
 def test_col_sum_is_four_running_sums(M, N):
     print(f"case: col_sum M={M} N={N}", flush=True)
