@@ -17,6 +17,7 @@
 // sums in a second kernel.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "internal.h"
@@ -355,11 +356,30 @@ __global__ __launch_bounds__(512) void gemm_direct(const __bf16* __restrict__ A,
       for (int y = 0; y < FN; ++y) o[SB != RFN ? 16 * y + i16 : FN * i16 + y] = acc[x][y][r];
     }
   __syncthreads();
-  for (int e = threadIdx.x; e < GM * GN; e += blockDim.x) {
-    const uint32_t i = e / GN, j = e % GN;
-    float s = red[(size_t)i * LD + j];
-    for (int w = 1; w < SK; ++w) s += red[((size_t)w * GM + i) * LD + j];
-    if (m0 + i < M && n0 + j < N) gemm_out(s, m0 + i, n0 + j, bias, act, Cf, Cb, ldc, beta);
+  // R outputs a thread at a time, so that their LDS reads overlap: a wave alone
+  // has 64 of a 64 x 64 tile, and one after the other they took longer than a
+  // product of few steps (4096 x 4096 x 64: 31 us, 28 so; 16384 x 512 x 2112 101, 99)
+  constexpr int R = 8;
+  const int nt = blockDim.x;
+  for (int e0 = threadIdx.x; e0 < GM * GN; e0 += R * nt) {
+    float s[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int e = min(e0 + q * nt, GM * GN - 1);
+      s[q] = red[e / GN * LD + e % GN];
+    }
+    for (int w = 1; w < SK; ++w)
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int e = min(e0 + q * nt, GM * GN - 1);
+        s[q] += red[(w * GM + e / GN) * LD + e % GN];
+      }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int e = e0 + q * nt;
+      const uint32_t i = m0 + e / GN, j = n0 + e % GN;
+      if (e < GM * GN && i < M && j < N) gemm_out(s[q], i, j, bias, act, Cf, Cb, ldc, beta);
+    }
   }
 }
 
@@ -568,21 +588,40 @@ hipError_t mlp_gemm(const MlpGemm& g, hipStream_t st) {
   // Direct kernel wherever both operands load in whole vectors and the splits
   // fit a workgroup. 32 x 32 tiles spread the network's own shapes over the
   // CUs; they read each operand once per 32 rows, so grids of 64 x 64 tiles
-  // that fill the chip several times over take those instead.
+  // that fill the chip several times over take those instead, from as many
+  // steps on as pay for the fewer waves: K > 256, or 192 where A's rows are the
+  // unit stride (more of the load unit's time); C of up to 32 columns (or rows)
+  // would be pad in half a tile, which long sums over such an A make up for.
+  // One or two steps of whole tiles stay with the staged kernel, whose four waves
+  // a tile store faster.
   // Measured, us a call, staged kernel (+ reduce) / 32 x 32 / 64 x 64 (M x N x K,
-  // T: both operands' rows unit-stride; a call costs 8 us to issue):
+  // T: A's rows, TT: both operands' rows unit-stride; a call costs 8 us to issue):
   //   273 x 512 x 2112      18.2 /  8.9 / 13.9
   //   1092 x 512 x 2112     40.8 / 18.0 / 21.4
-  //   2112 x 512 x 1092 T    107 / 18.2 / 26.3
+  //   2112 x 512 x 1092 TT   107 / 18.2 / 26.3
   //   4368 x 512 x 512      40.0 / 16.2 / 23.3   (552 tiles of 64 x 64)
-  //   8192 x 512 x 512         - / 23.5 / 27.0   (1024)
-  //   16384 x 512 x 512     81.6 / 42.6 / 38.0   (2048)
-  //   16384 x 512 x 2112     200 /  182 /  107   (2048)
-  //   2112 x 512 x 16384 T  1486 /  236 /  185   (264)
+  //   8192 x 512 x 512      29.3 / 22.0 / 23.1   (1024)
+  //   16384 x 512 x 64      14.7 / 15.5 / 18.1   (2048)
+  //   16384 x 512 x 128     19.7 / 18.4 / 20.9
+  //   16384 x 512 x 512     50.0 / 40.1 / 33.9
+  //   16384 x 512 x 2112     187 /  163 /   99
+  //   4096 x 4096 x 32      19.7 / 23.4 / 25.9   (4096)
+  //   4096 x 4096 x 128     31.0 / 28.6 / 31.6
+  //   4096 x 4096 x 192 T   83.9 / 38.1 / 34.4
+  //   4096 x 4096 x 384     71.4 / 58.5 / 46.3
+  //   100000 x 16 x 64      12.4 / 10.3 / 14.3   (1563, three quarters of each pad)
+  //   70000 x 32 x 2112      329 /   66 /   77   (1094, half pad; T 669 / 106 / 89)
+  //   2112 x 512 x 16384 TT 1486 /  236 /  185   (264)
   if (splits <= 8) {
     const uint64_t tiles64 = (uint64_t)((g.M + 63) / 64) * ((g.N + 63) / 64);
-    if (tiles64 >= 1024 && fits(4)) return direct_pick<4>(g, sa, sb, splits, kchunk, st);
-    if ((g.M + 31) / 32 <= 65535 && fits(2)) return direct_pick<2>(g, sa, sb, splits, kchunk, st);
+    const bool many = tiles64 >= 1024;
+    if (many && fits(4) && g.K > (sa == KF ? 256 : 191) &&
+        (std::min(g.M, g.N) > 32 || (sa != KF && g.K >= 1024)))
+      return direct_pick<4>(g, sa, sb, splits, kchunk, st);
+    const bool staged = many && g.K >= TK && g.K <= 2 * TK && g.M % TM == 0 && g.N % TN == 0 &&
+                        fits(2) && sa == KF && sb == RF;
+    if (!staged && (g.M + 31) / 32 <= 65535 && fits(2))
+      return direct_pick<2>(g, sa, sb, splits, kchunk, st);
   }
   float* part = nullptr;
   if (splits > 1) {

@@ -82,6 +82,14 @@ def test_gemm_direct_equals_staged(M, N, K):
             assert t.equal(got[0][0], got[1][0]) and t.equal(got[0][1], got[1][1]), (a_t, b_t)
 
 
+@pytest.mark.parametrize("M,N,K", [(2056, 2048, 264), (2048, 2112, 200), (2048, 2048, 64),
+                                   (2048, 2048, 40), (32776, 32, 1032), (65544, 24, 328)])
+def test_gemm_tile_choices_equal_staged(M, N, K):
+    """Either side of the lines between 64 x 64 tiles, 32 x 32 tiles and the staged
+    kernel: many tiles, with few and many steps, C of up to 32 columns."""
+    test_gemm_direct_equals_staged(M, N, K)
+
+
 @pytest.mark.parametrize("M,N", [(64, 64), (33, 70)])  # the register and the staged kernel
 def test_gemm_of_an_empty_sum_is_its_epilogue(M, N):
     """K = 0: no operand is read, C is the bias (and beta times what it held)."""
