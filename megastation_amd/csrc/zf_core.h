@@ -472,8 +472,11 @@ __device__ __forceinline__ void zf_apply(const float2* A, uint32_t U, uint32_t B
   // lanes in neighbour antennas) every lane costs one (65). So do W's stores,
   // which is why the antennas are the product's rows: sixteen users of an antenna
   // a quarter wave. 256 x 32 x 273: 37.1 -> 34.4 us, 256 x 64: 122 -> 117. With
-  // eight user tiles the users stay the rows (as above, 4 % more time).
-  constexpr bool BROW = UT <= 4, QUAD = BROW && !A_LDS;
+  // eight user tiles the users stay the rows (as above, 4 % more time); one tile
+  // keeps the operand's order of loads, its one wave a group having nothing to hide
+  // the exchange behind (W = X A, 273 groups of 64 x 8: 5.7 us with it, 5.4
+  // without, 5.3 with the users as rows; 2000 of 128 x 16: 15.0, 15.7, 19.3).
+  constexpr bool BROW = UT <= 4, QUAD = BROW && !A_LDS && UT > 1;
   auto prod = [](float av, float gv, v4f acc) {
     return BROW ? mfma4(av, gv, acc) : mfma4(gv, av, acc);
   };
