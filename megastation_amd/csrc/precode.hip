@@ -233,18 +233,17 @@ hipError_t precode_run(const PrecodeArgs& a, uint64_t G, uint32_t ntile, hipStre
   // about 4/3 rounds of four waves a SIMD of them. us, ranges / dealt: 128 x 8
   // 17.6 / 15.7, 256 x 16 33.2 / 31.0, 300 x 24 48.7 / 43.4; but 128 x 16 19.0 /
   // 20.4, 256 x 24 34.7 / 37.5. Otherwise, with antenna blocks off a multiple of
-  // four, ranges that end with their groups: 160 x 32 35.6 / 28.2, 96 x 16 17.5 /
-  // 15.8 (128 x 16, four blocks: 19.0 / 19.7).
+  // four, ranges that end with their groups if they are waves enough: 160 x 32
+  // 35.6 / 28.2, 96 x 16 17.5 / 15.8; but 128 x 16, four blocks, 19.0 / 19.7, and
+  // 219 x 52, 42 groups of 14 tiles, 1176 waves instead of 2048, 32.8 / 35.2.
   if (J <= 2 || (J == 4 && G * nab >= waves) || (J == 6 && G * nab >= waves + waves / 4)) {
     nrange = G;
     phases = J > 4 ? 1 : std::max<uint64_t>(2, (8 * waves / 3 + G * nab / 2) / (G * nab));
     phases = std::min<uint64_t>(phases, ntile);
-  } else if (nab % 4 && 4 * G * nab >= waves) {
-    for (uint64_t k = std::min<uint64_t>(ntile, (2 * waves + G * nab) / (2 * G * nab)); k > 0; --k)
-      if (ntile % k == 0) {
-        nrange = k * G;
-        break;
-      }
+  } else if (nab % 4) {
+    uint64_t k = std::min<uint64_t>(ntile, (2 * waves + G * nab) / (2 * G * nab));
+    while (k > 0 && ntile % k) --k;
+    if (5 * k * G * nab >= 4 * waves) nrange = k * G;
   }
   const uint64_t grid = (nab * nrange * std::max<uint64_t>(1, phases) + 3) / 4;
   if (grid > 0xffffffu) {  // a launch's threads: 32 bits
