@@ -154,7 +154,7 @@ __global__ __launch_bounds__(512, eq_wide_waves(MT, 8)) void eq_cells_wide(const
   const uint32_t u = unit - prefix[c];
   const uint32_t g = u / p.chunks;
   with_order(p.Q, [&](auto q) {
-    eq_wide_unit<MT, KS, 8, decltype(q)::value>(p, 0, g, u - g * p.chunks, p.tiles_per_wg, red);
+    eq_wide_unit<MT, KS, 8, decltype(q)::value, true>(p, 0, g, u - g * p.chunks, p.tiles_per_wg, red);
   });
 }
 

@@ -43,7 +43,12 @@ template <int MT, int NW>
 using EqWideRed = float[2][NW][MT][2][4][64];
 
 // Chunk c of tc column tiles of group g of a slot, by one workgroup of NW waves.
-template <int MT, int KS, int NW, int Q>
+// The operand sums make NaN of an infinite sample (K1 - K3 cancels), and overflow
+// on one within a factor of two of the largest float, where the four products
+// give a signed infinity or a finite value. With FOUR a lane that has stored a
+// symbol that is not finite forms its symbols of the unit again that way, after
+// the loop, and stores those with such an operand or result.
+template <int MT, int KS, int NW, int Q, bool FOUR = false>
 __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, uint32_t g,
                                              uint32_t c, uint32_t tc, EqWideRed<MT, NW>& red) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -89,6 +94,7 @@ __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, u
 
   // outputs of column tile t from partial buffer b: wave w adds up, demods and
   // stores outputs (m, r) = pi / 4, pi % 4 for pi = w, w + NW, ...
+  bool finite = true;
   auto finish = [&](uint32_t t, int b) {
     const EqCol col = eq_col<Q>(p, slot, g, t);
 #pragma unroll
@@ -101,6 +107,7 @@ __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, u
         im += red[b][j][m][1][r][lane];
       }
       const uint32_t u = 16 * m + 4 * q4 + r;
+      if constexpr (FOUR) finite &= fabsf(re) + fabsf(im) < __builtin_inff();
       if (col.valid && u < U) {
         store_llrs<Q>(p, col.rows + u * p.ue_stride, col.ls, re, im);
         if (col.xrow) col.xrow[(uint64_t)u * N] = make_float2(re, im);
@@ -182,6 +189,29 @@ __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, u
     buf ^= 1;
   }
   finish(t1 - 1, buf ^ 1);
+  if constexpr (FOUR) {
+    if (finite) return;
+    for (uint32_t t = t0; t < t1; ++t) {
+      const EqCol col = eq_col<Q>(p, slot, g, t);
+      if (!col.valid) continue;
+      const uint32_t n = 16 * t + i16, sym = group_sym(p, n, nk);
+      const float2* yc = p.y + slot * p.y_slot + sym * p.y_sym + k0 + (n - sym * nk);
+      for (int pi = w; pi < 4 * MT; pi += NW) {
+        const uint32_t u = 16 * (pi / 4) + 4 * q4 + pi % 4;
+        if (u >= U) continue;
+        float re = 0.f, im = 0.f, top = 0.f;
+        for (uint32_t b = 0; b < B; ++b) {
+          const float2 v = W[u + (uint64_t)b * U], yv = yc[(uint64_t)b * N];
+          re = fmaf(-v.y, yv.y, fmaf(v.x, yv.x, re));
+          im = fmaf(v.y, yv.x, fmaf(v.x, yv.y, im));
+          top = fmaxf(top, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(yv.x), fabsf(yv.y))));
+        }
+        if (top < 0x1p120f && fabsf(re) + fabsf(im) < __builtin_inff()) continue;
+        store_llrs<Q>(p, col.rows + u * p.ue_stride, col.ls, re, im);
+        if (col.xrow) col.xrow[(uint64_t)u * N] = make_float2(re, im);
+      }
+    }
+  }
 }
 
 }  // namespace detail

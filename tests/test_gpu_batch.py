@@ -172,6 +172,55 @@ def test_batch_wide_plans_of_every_user_tile_count(tmp_path, monkeypatch):
     test_batch_wide_plans_agree_for_every_chunk_count(tmp_path, monkeypatch)
 
 
+@pytest.mark.parametrize("cell", [
+    (8, 64, 60, 12, 4, "standalone"), (16, 128, 50, 12, 2, "standalone"),
+    (32, 256, 30, 12, 6, "standalone"), (50, 96, 31, 16, 8, "standalone")])
+def test_batch_infinite_samples(cell, monkeypatch):
+    """A received sample of infinite (or overflowing) parts: its column's symbols
+    are the four real products' sums, infinities with their signs or NaN where
+    they cancel; every other column keeps its bits."""
+    print(f"case: batch infinite samples {cell}", flush=True)
+    t = torch()
+    monkeypatch.setitem(globals(), "CELLS", [cell])
+    U, B, N, sg, Q, _ = cell
+    c, = _make_cells(seed=21, S=3)
+    b = m.Batch([c])
+    b.run()
+    t.cuda.synchronize()
+    clean, llr = host_c64(c["xhat"]).reshape(3, U, N), host_u16(c["llr"]).reshape(3, U, -1).copy()
+    y = c["y"].cpu().numpy().reshape(3, B, N).copy()
+    y[0, 5, 7] = complex(np.inf, 0.5)
+    y[1, B - 1, 0] = complex(0.25, -np.inf)
+    y[2, 0, N - 1] = complex(-np.inf, np.inf)
+    y[2, B // 2, 20] = complex(3e38, -3e38)  # yi - yr overflows, the products may not
+    c["y"].copy_(t.from_numpy(y).reshape(c["y"].shape))
+    b.run()
+    t.cuda.synchronize()
+    b.close()
+    got = host_c64(c["xhat"]).reshape(3, U, N)
+    got_llr = host_u16(c["llr"]).reshape(3, U, -1)
+    w = np.repeat(host_c64(c["w"]).reshape(-1, B, U), sg, axis=0)[:N].astype(np.complex128)
+    hit = [(0, 7), (1, 0), (2, N - 1), (2, 20)]
+    for s, k in hit:
+        x, wk = y[s, :, k].astype(np.complex128), w[k]                       # [B], [B][U]
+        with np.errstate(invalid="ignore"):
+            re = (wk.real * x.real[:, None] - wk.imag * x.imag[:, None]).sum(0)
+            im = (wk.real * x.imag[:, None] + wk.imag * x.real[:, None]).sum(0)
+        for g, e in ((got[s, :, k].real, re), (got[s, :, k].imag, im)):
+            assert np.array_equal(np.isnan(g), np.isnan(e)), (s, k)
+            inf = np.isinf(e)
+            assert (g[inf] == e[inf]).all(), (s, k)
+            fin = np.isfinite(e) & (np.abs(e) < 3e38)
+            assert (np.abs(g[fin] - e[fin]) <= 1e-4 * np.abs(e[fin]).max(initial=0)).all(), (s, k)
+    same = np.ones((3, N), bool)
+    for s, k in hit:
+        same[s, k] = False
+        got_llr[s, :, k * Q:(k + 1) * Q] = llr[s, :, k * Q:(k + 1) * Q]
+    for s in range(3):
+        assert np.array_equal(got[s][:, same[s]], clean[s][:, same[s]])
+    assert np.array_equal(got_llr, llr)
+
+
 @pytest.mark.parametrize("saved", [
     "stream MT=2 waves/CU=12",          # the candidate set before the wide form
     "wide MT=1 KS=4 chunks=4294967295",  # more chunks than 32-bit sums hold
