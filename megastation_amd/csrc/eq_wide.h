@@ -1,16 +1,17 @@
-// FP32 equalize + demod for wide cells (up to 64 users, 128 or 256
-// antennas, e.g. 256 x 32): the antennas are split over the four or eight
-// waves of a workgroup, each wave keeps its slice of W_g in registers for
-// the whole unit (16, 32 or 64 users: one, two or four 16-user tiles), and
-// the complex products take three real MFMAs instead of four. Shared by the
-// stand-alone kernels (equalize_wide.hip) and the batch's (batch.hip).
+// FP32 equalize + demod for wide cells (up to 64 users and 256 antennas, e.g.
+// 256 x 32): the antennas are split over the four or eight waves of a
+// workgroup, each wave keeps its slice of W_g in registers for the whole unit
+// (16, 32 or 64 users: one, two or four 16-user tiles), and the complex
+// products take three real MFMAs instead of four. Shared by the stand-alone
+// kernels (equalize_wide.hip: from 128 antennas) and the batch's (batch.hip:
+// from 64, always on eight waves).
 //
 // Unit = (slot, group, chunk of TC column tiles of 16 (symbol, subcarrier)
 // columns). Wave w owns antennas 4*KS*w .. 4*KS*(w+1)-1 (KS steps of 4) and
 // computes, for every column tile of the unit, the partial products over its
-// antennas for all 16*MT users; the four partial tiles meet in LDS (double
+// antennas for all 16*MT users; the waves' partial tiles meet in LDS (double
 // buffered, one barrier per tile) and each wave adds up (in wave order),
-// demodulates and stores a quarter of the tile's outputs.
+// demodulates and stores its share of the tile's outputs.
 //
 // Products (Gauss): with W = Wr + i Wi and y = yr + i yi, per 4-antenna step
 // and 16-user x 16-column tile
@@ -61,8 +62,8 @@ __device__ __forceinline__ void eq_wide_unit(const EqParams& p, uint32_t slot, u
   const uint32_t t1 = min(t0 + tc, (ncol + 15) / 16);
   if (t0 >= t1) return;  // a chunk past a partial group: uniform
 
-  // ---- this wave's W slice: Wr, Wi per (user tile, step); Wr + Wi is formed
-  // at each use (one add per MFMA triple saves a third of the slice's
+  // ---- this wave's W slice: Wr, Wi per (user tile, step); Wr + Wi is formed for
+  // each column tile (one add per MFMA triple saves a third of the slice's
   // registers) -----------------------------------------------------------------
   const float2* W = p.csi + slot * p.csi_slot + (uint64_t)g * U * B;
   const uint32_t bw = 4 * KS * w;  // first antenna of the slice
