@@ -236,7 +236,10 @@ hipError_t precode_run(const PrecodeArgs& a, uint64_t G, uint32_t ntile, hipStre
   // four, ranges that end with their groups if they are waves enough: 160 x 32
   // 35.6 / 28.2, 96 x 16 17.5 / 15.8; but 128 x 16, four blocks, 19.0 / 19.7, and
   // 219 x 52, 42 groups of 14 tiles, 1176 waves instead of 2048, 32.8 / 35.2.
-  if (J <= 2 || (J == 4 && G * nab >= waves) || (J == 6 && G * nab >= waves + waves / 4)) {
+  const bool dealt =
+      J <= 2 || (J == 4 && G * nab >= waves) || (J == 6 && G * nab >= waves + waves / 4);
+  constexpr uint64_t kMaxWaves = 4 * 0xffffffull;  // a launch's threads: 32 bits
+  if (dealt && G * nab <= kMaxWaves / 2) {
     nrange = G;
     phases = J > 4 ? 1 : std::max<uint64_t>(2, (8 * waves / 3 + G * nab / 2) / (G * nab));
     phases = std::min<uint64_t>(phases, ntile);
@@ -246,7 +249,7 @@ hipError_t precode_run(const PrecodeArgs& a, uint64_t G, uint32_t ntile, hipStre
     if (5 * k * G * nab >= 4 * waves) nrange = k * G;
   }
   const uint64_t grid = (nab * nrange * std::max<uint64_t>(1, phases) + 3) / 4;
-  if (grid > 0xffffffu) {  // a launch's threads: 32 bits
+  if (4 * grid > kMaxWaves) {
     *why = "grid too large";
     return hipErrorInvalidValue;
   }

@@ -198,6 +198,19 @@ def test_bad_ldpc_arguments_rejected_before_launch():
     assert call(num_cb=0) == m.MEGA_OK          # nothing to decode
 
 
+@pytest.mark.parametrize("N,sg,B,U", [(2**28, 1, 64, 4), (2**27, 1, 300, 8), (2**26, 2, 256, 16),
+                                      (2**26, 1, 300, 24), (2**26, 1, 200, 32)])
+def test_precode_takes_any_number_of_groups(N, sg, B, U):
+    """Groups beyond what a launch of a wave a group holds: as above."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("would launch on stand-in pointers")
+    p = ctypes.c_void_p(4096).value
+    d = m.PrecodeDesc(B, U, N, sg, 1, N, 0, p, p, U * N, p, B * N)
+    assert m.lib().mega_precode_syms(ctypes.byref(d), None) == m.MEGA_ERR_HIP
+    assert "grid too large" not in m.last_error()
+
+
 def _mlp_layers():
     """Two chained layers of stand-in pointers (nothing is launched)."""
     from megastation_amd import learned
