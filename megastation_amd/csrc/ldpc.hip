@@ -109,7 +109,16 @@ static_assert(ldpc::kBg1Edges <= kMaxEdges && ldpc::kBg2Edges <= kMaxEdges, "edg
 using KEdge = const __attribute__((address_space(4))) LdpcParams::Edge*;
 static_assert(offsetof(LdpcParams, edge) % 4 == 0 && sizeof(LdpcParams) <= 4096, "kernarg");
 
-template <int BG, int NB>  // NB: code blocks of a workgroup
+// Rows of the instances for codes of few parity rows (high rates). Base graph 1's
+// four rows of 19 edges are most of their work, and the registers of the other
+// rows' messages hold those rows' addresses, where the whole graph's instance
+// forms them again, four at a time; and there are fewer rows to pass by. 64 code
+// blocks of Zc 44, 8 iterations, whole graph's instance / this one (and as it was
+// with two waves a SIMD): base graph 1, 4 rows 52.3 / 38.5 us (44.3), 24 rows 108 /
+// 97.7 (113); base graph 2, 4 rows 24.0 / 20.7 (22.4).
+constexpr int few_rows(int bg) { return bg == 1 ? 24 : 12; }
+
+template <int BG, int NB, int ROWS>  // NB: code blocks of a workgroup
 __global__ __launch_bounds__(768, 3) void ldpc_decode(const LdpcParams p) {
   using G = Bg<BG>;
   extern __shared__ float L[];  // NB times (kb + mb) * zc negated LLRs, then the bit words
@@ -141,16 +150,16 @@ __global__ __launch_bounds__(768, 3) void ldpc_decode(const LdpcParams p) {
   __syncthreads();
 
   // compressed messages of this thread's check in every row
-  float m1[G::rows], m2[G::rows];
+  float m1[ROWS], m2[ROWS];
   constexpr SignWords<BG> SW;
   uint32_t pk[SW.words];  // sign bits (a row's last edge lowest) and index of the minimum
 #pragma unroll
-  for (int r = 0; r < G::rows; ++r) m1[r] = m2[r] = 0.f;
+  for (int r = 0; r < ROWS; ++r) m1[r] = m2[r] = 0.f;
 #pragma unroll
   for (int w = 0; w < SW.words; ++w) pk[w] = 0u;
 
   for (uint32_t it = 0; it < p.iters; ++it) {
-    static_for<0, G::rows>([&](auto rc) {
+    static_for<0, ROWS>([&](auto rc) {
       constexpr int r = decltype(rc)::value;
       constexpr int e0 = G::start(r), deg = G::start(r + 1) - G::start(r);
       // uniform; a count the compiler cannot see through, so that it compares
@@ -167,21 +176,21 @@ __global__ __launch_bounds__(768, 3) void ldpc_decode(const LdpcParams p) {
         uint64_t ka = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
         __asm__ __volatile__("" : "+s"(ka));
         const KEdge ew = reinterpret_cast<KEdge>(ka + offsetof(LdpcParams, edge));
-        constexpr bool PAIR = deg <= kPairDeg;
+        constexpr bool PAIR = deg <= kPairDeg, HELD = PAIR || ROWS < G::rows;
         constexpr int W = SW.word[r], sh0 = 16 * SW.half[r], ibit = PAIR ? sh0 + 12 : 24;
         auto addr = [&](KEdge t, int e) {  // LDS byte address
           return (z4 >= t[e0 + e].wrap ? hi : lo) + t[e0 + e].base;
         };
         uint32_t vi[deg];
         float lv[deg];
-        if constexpr (PAIR) {
+        if constexpr (HELD) {
 #pragma unroll
           for (int e = 0; e < deg; ++e) vi[e] = addr(ew, e);
         }
 #pragma unroll
         for (int e = 0; e < deg; ++e) {
-          lv[e] = *reinterpret_cast<const float*>(Lb + (PAIR ? vi[e] : addr(ew, e)));
-          if (!PAIR && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          lv[e] = *reinterpret_cast<const float*>(Lb + (HELD ? vi[e] : addr(ew, e)));
+          if (!HELD && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         // Q and R are negated as L is. R_old of edge e: alpha*min2 at the old
         // minimum's edge, alpha*min1 elsewhere (both >= +0), negated where its
@@ -221,7 +230,7 @@ __global__ __launch_bounds__(768, 3) void ldpc_decode(const LdpcParams p) {
         // the widest rows form their addresses again, four at a time, instead
         // of holding them
         uint64_t kb = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
-        if constexpr (!PAIR) __asm__ __volatile__("" : "+s"(kb));
+        if constexpr (!HELD) __asm__ __volatile__("" : "+s"(kb));
         const KEdge ew2 = reinterpret_cast<KEdge>(kb + offsetof(LdpcParams, edge));
 #pragma unroll
         for (int e = 0; e < deg; ++e) {
@@ -233,9 +242,9 @@ __global__ __launch_bounds__(768, 3) void ldpc_decode(const LdpcParams p) {
           const float mag = least ? n2 : n1;
           const float rnew = __uint_as_float((__float_as_uint(mag) & 0x7fffffffu) |
                                              (__float_as_uint(q[e]) & 0x80000000u));
-          *reinterpret_cast<float*>(Lb + (PAIR ? vi[e] : addr(ew2, e))) =
+          *reinterpret_cast<float*>(Lb + (HELD ? vi[e] : addr(ew2, e))) =
               __builtin_fmaf(rnew, ps, q[e]);
-          if (!PAIR && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+          if (!HELD && e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         m1[r] = n1;
         m2[r] = n2;
@@ -313,8 +322,13 @@ hipError_t launch_ldpc_decode(const LdpcArgs& a, hipStream_t st, const char** wh
   const uint32_t nb = ldpc_blocks(a.zc, lds, a.num_cb);
   lds *= nb;
   const dim3 grid((a.num_cb + nb - 1) / nb), block((nb * a.zc + 63) / 64 * 64);
-  void (*fn)(const LdpcParams) = a.bg == 1 ? nb == 1 ? ldpc_decode<1, 1> : ldpc_decode<1, 2>
-                                 : nb == 1 ? ldpc_decode<2, 1> : ldpc_decode<2, 2>;
+  auto pick = [&](auto graph) -> void (*)(const LdpcParams) {
+    constexpr int BG = decltype(graph)::value, FEW = few_rows(BG), ALL = Bg<BG>::rows;
+    if (a.mb <= FEW) return nb == 1 ? ldpc_decode<BG, 1, FEW> : ldpc_decode<BG, 2, FEW>;
+    return nb == 1 ? ldpc_decode<BG, 1, ALL> : ldpc_decode<BG, 2, ALL>;
+  };
+  const auto fn = a.bg == 1 ? pick(std::integral_constant<int, 1>{})
+                            : pick(std::integral_constant<int, 2>{});
   if (lds > 65536) {
     e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

@@ -100,6 +100,18 @@ def test_more_code_blocks_than_cus_match_oracle(bg, zc, mb, half, n_cb):
     assert np.all(out[:, words:] == 0xFFFFFFFF)
 
 
+@pytest.mark.parametrize("bg,zc,mb", [(1, 72, 4), (1, 60, 24), (1, 60, 25), (2, 72, 4),
+                                      (2, 60, 12), (2, 60, 13)])
+def test_instances_for_few_rows_match_oracle(bg, zc, mb):
+    """Either side of the row counts up to which a smaller instance decodes."""
+    test_decoder_matches_oracle_on_noisy_code_blocks(bg, zc, mb, False)
+
+
+@pytest.mark.parametrize("bg,zc,mb", [(1, 320, 24), (2, 288, 12), (2, 288, 5)])
+def test_instances_for_few_rows_in_pairs_match_oracle(bg, zc, mb):
+    test_more_code_blocks_than_cus_match_oracle(bg, zc, mb, True, 259)
+
+
 def _decode_numpy(llr, bg, zc, mb, iters, alpha):
     """The layered schedule in numpy FP32 with the kernel's rule for NaN: not
     negative, never the minimum, min2 down to min1 (llr [n][(kb + mb) * zc])."""
