@@ -355,12 +355,14 @@ typedef struct {
 typedef struct mega_batch *mega_batch_t;
 
 /* Plans a batch: cells are grouped into kernel classes (ZF by users rounded
- * to 16-user tiles; equalize by antenna count), each equalize class's tile
- * plan and the launch schedule are chosen by timing the candidates on these
- * buffers (the autotuner: runs the batch several times, so outputs are
- * overwritten), and the chosen launches are captured into one hipGraph.
- * tune_path (optional) caches tuned plans across processes (a text file,
- * appended). Buffers are bound: run the handle on the same buffers. */
+ * to 16-user tiles; equalize by antenna count and user tiles, small cells of
+ * one antenna count together), each equalize class's tile plan and the launch
+ * schedule are chosen by timing the candidates on these buffers (the
+ * autotuner: runs the batch several times, so outputs are overwritten), and
+ * the chosen launches are captured into one hipGraph. tune_path (optional)
+ * caches tuned plans across processes (a text file, appended; a line that is
+ * no candidate of its class is measured again). Buffers are bound: run the
+ * handle on the same buffers. */
 int mega_batch_create(const mega_cell_desc *cells, uint32_t num_cells,
                       const char *tune_path, mega_batch_t *out);
 /* ZF + equalize + demod of every cell: one hipGraphLaunch on stream. */
